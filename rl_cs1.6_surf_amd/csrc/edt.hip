@@ -20,12 +20,14 @@
 // sum of per-axis squares equals cell^2 * D exactly, so the result is
 // bit-identical to the reference's bake.
 //
-// The y and z passes have two implementations with identical results: the
-// envelope walk above (one thread per line) for passes with many lines, and
-// a windowed exact search per output (edt_window) for passes with few.
+// The passes have two implementations with identical results: tiles of lines
+// staged in LDS, 16-bit or 32-bit squares (edt_pack, edt_tile), wherever the y
+// and z lines fit; and, for longer lines, the walk above (edt_rows, edt_cols,
+// edt_slabs; one thread per y or z line).
 //
 // Scratch: two int32 planes of the grid and one uint64 envelope stack per
-// line (~16 bytes per voxel, sdfr_edt_workspace_bytes).
+// line (~16 bytes per voxel, sdfr_edt_workspace_bytes); the tiles use at most
+// 13 bytes per voxel of it.
 
 #include <hip/hip_runtime.h>
 #include <hip/hip_fp16.h>
@@ -33,6 +35,9 @@
 #include <stdint.h>
 #include <stdio.h>
 #include <stdarg.h>
+#include <string.h>
+
+#include <type_traits>
 
 #include "../../include/sdfr.h"
 
@@ -226,101 +231,408 @@ __global__ __launch_bounds__(256) void edt_slabs(const int32_t* __restrict__ f, 
                   fout ? fout + line : nullptr, hout ? hout + line : nullptr, cell2);
 }
 
-// ---------------------------------------------------------- windowed passes --
-// The y and z passes again, as a search per output instead of a walk per
-// line: D(q) = min over p of f(p) + (q - p)^2, with the pads f(-1) = f(n) = 0.
-// Starting from p = q (which gives f(q)), the candidates at distance d on
-// either side are tried for d = 1, 2, ... while d^2 < best: a candidate at
-// distance d adds at least d^2, so none further out can win, and the answer
-// is exact. The pads bound best by min(q + 1, n - q)^2, so the search never
-// leaves [-1, n]. A workgroup stages T whole lines (a tile of neighbouring
-// columns) in LDS, entry (p + 1) * T + c for line c, and a wave works on
-// 64 / T consecutive outputs of all T lines, whose searches are about equally
-// long (neighbouring voxels have similar distances). The work is the sum of
-// the distances in voxels; tens of thousands of waves are in flight instead
-// of one per 64 lines.
+// ------------------------------------------------------------- tiled passes --
+// The transform in three kernels that move 7.5 bytes a voxel and the output
+// between them (a byte of occupancy, a quarter byte of packed bits each way,
+// 16-bit squares each way). A pass searches, for every output q of a line,
+// D(q) = min over p of f(p) + (q - p)^2 over whole lines staged in LDS.
 //
-// Lines of tile (bx, by): pass y (AXIS 1) lines (z = by, x), element p at
-// (z*ny + p)*nx + x; pass z (AXIS 2) lines (y, x), y in [by*ty, by*ty + ty),
-// element p at (p*ny + y)*nx + x. In both, x in [bx*tx, bx*tx + tx), T = tx*ty.
-template <int AXIS, bool LAST>
-__global__ __launch_bounds__(256) void edt_window(const int32_t* __restrict__ f,
-                                                  int32_t* __restrict__ out,
-                                                  float* __restrict__ fout,
-                                                  __half* __restrict__ hout, int nx, int ny,
-                                                  int nz, int tx, int ty, double cell2) {
-    extern __shared__ int32_t s[];
-    const int T = tx * ty;
-    const int n = AXIS == 1 ? ny : nz;
-    const int64_t stride = AXIS == 1 ? (int64_t)nx : (int64_t)nx * ny;
-    const int x0 = blockIdx.x * tx;
-    const int by = blockIdx.y;
-    // element p of tile line c, or -1 for a line outside the grid
-    auto line_base = [&](int c) -> int64_t {
-        const int x = x0 + c % tx;
-        if (x >= nx) return -1;
-        if (AXIS == 1) return (int64_t)by * ny * nx + x;
-        const int y = by * ty + c / tx;
-        return y < ny ? (int64_t)y * nx + x : -1;
-    };
-    for (int i = threadIdx.x; i < (n + 2) * T; i += blockDim.x) {
-        const int p = i / T - 1, c = i - (i / T) * T;
-        const int64_t b = line_base(c);
-        s[i] = (p < 0 || p >= n || b < 0) ? 0 : f[b + (int64_t)p * stride];
+//   * Only what can still win is kept. The solid layer above and below the
+//     grid bounds every distance along z by min(z + 1, nz - z), and a value
+//     f(p) at plane p can only take part in one of them if it is below
+//         max over q of min(q + 1, nz - q)^2 - (q - p)^2 = (p + 1)(nz - p):
+//     the first bound grows with q, the second falls, they meet at
+//     2q = nz - 1. So values of the x and y passes are clamped there (z_cap)
+//     without changing a result, which also bounds the y search by
+//     sqrt(z_cap); for nz <= 509 the squares fit 16 bits (two voxels a
+//     register, v_pk_add_u16 saturating and v_pk_min_u16) and the distances
+//     along x a byte.
+//   * A thread takes kBlk consecutive outputs of a line (two lines when
+//     packed) in registers and reads each candidate once for all of them.
+//   * Candidates come in chunks of kBlk rows, nearest first, on both sides,
+//     until even a zero in the next chunk could not win (its nearest row is
+//     kBlk(c - 1) + 1 away); a chunk whose smallest value (kept per chunk and
+//     line) cannot win at that distance either is skipped. Neighbouring lines
+//     agree about both, so on the scenes measured a wave searches ~4 of a
+//     line's 128 chunks.
+//
+// What bounds it is vector issue (the searches) and, at their start, the wait
+// for the tile: at 256x256x128 voxels 5.5 + 32 + 26 us (36 + 98 + 62 us for a
+// wave per row and a search per output), at 1024x1024x256 125 + 750 + 622 us
+// (3049 + 4881 + 3207 us for the wave per row and the walk per line); the
+// bytes alone take 14 and 430 us at a copy's 4.7 TB/s. 8 outputs a thread
+// beat 16 (40 + 32, 887 + 831 us) as they leave twice the waves in flight;
+// tiles 32 words wide beat 64, of which fewer fit a CU (33 + 27, 1077 +
+// 785 us); 1024 threads beat 512 in the y pass, whose tiles fill the LDS
+// (749 against 930 us), and lose in the z pass (741 against 622).
+typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+
+constexpr int kBlk = 8;
+constexpr int kThreadsY = 1024, kThreadsZ = 512;
+
+template <typename V> struct Word;
+template <> struct Word<u16x2> {   // two voxels, 16-bit squares
+    typedef uint16_t Plane;
+    static constexpr int kVox = 2;
+    static constexpr uint32_t kMax = 0xffffu;
+    static __device__ __forceinline__ u16x2 splat(uint32_t v) {
+        const unsigned short h = (unsigned short)v;
+        return u16x2{h, h};
+    }
+    static __device__ __forceinline__ u16x2 add(u16x2 a, u16x2 b) { return __builtin_elementwise_add_sat(a, b); }
+    static __device__ __forceinline__ bool any_less(u16x2 a, u16x2 b) {
+        return __builtin_bit_cast(uint32_t, __builtin_elementwise_sub_sat(b, a)) != 0u;
+    }
+    static __device__ __forceinline__ uint32_t get(u16x2 v, int i) { return i ? v.y : v.x; }
+};
+template <> struct Word<uint32_t> {   // one voxel
+    typedef uint32_t Plane;
+    static constexpr int kVox = 1;
+    static constexpr uint32_t kMax = 0x3fffffffu;   // kMax + any (q - p)^2 stays below 2^32
+    static __device__ __forceinline__ uint32_t splat(uint32_t v) { return v; }
+    static __device__ __forceinline__ uint32_t add(uint32_t a, uint32_t b) { return a + b; }
+    static __device__ __forceinline__ bool any_less(uint32_t a, uint32_t b) { return a < b; }
+    static __device__ __forceinline__ uint32_t get(uint32_t v, int) { return v; }
+};
+
+// What a tile holds per word in LDS: the squares, or in the packed y pass the
+// two distances along x in a byte each, squared when they are read.
+template <typename V, bool Z> struct Cell {
+    typedef V T;
+    static __device__ __forceinline__ V open(T c) { return c; }
+    static __device__ __forceinline__ T shut(V v) { return v; }
+    static __device__ __forceinline__ V value(V v) { return v; }
+    static __device__ __forceinline__ V far() { return Word<V>::splat(Word<V>::kMax); }
+};
+template <> struct Cell<u16x2, false> {
+    typedef uint16_t T;
+    static __device__ __forceinline__ u16x2 open(T c) {
+        return __builtin_bit_cast(u16x2, (uint32_t)__builtin_amdgcn_perm(0u, c, 0x0c010c00u));
+    }
+    static __device__ __forceinline__ T shut(u16x2 v) { return (T)(v.x | (v.y << 8)); }
+    static __device__ __forceinline__ u16x2 value(u16x2 v) { return v * v; }
+    static __device__ __forceinline__ u16x2 far() { return Word<u16x2>::splat(255u); }
+};
+
+// Block b runs on XCD b % 8; give each XCD a contiguous run of tiles, so that
+// tiles beside each other along x, which share 128-byte lines, share an L2.
+__device__ __forceinline__ int64_t xcd_tile(int64_t b, int64_t n) {
+    const int64_t q = n >> 3, rem = n & 7, x = b & 7;
+    return x * q + (x < rem ? x : rem) + (b >> 3);
+}
+
+// Pass x: the occupancy as bits. Per 32 voxels of a row (voxels past its end
+// count as solid: they are the padding): the bits, the distance from the
+// first voxel back to the last solid before it (low 16 bits) and from the
+// last voxel to the first solid after it (high 16). A quarter byte a voxel,
+// from which the y pass forms any voxel's distance with two bit scans. Laid
+// out [nz][words][ny], so that a tile's rows are consecutive.
+// R rows of a block are packed into LDS, then each (row, word) looks outward
+// for the nearest word that holds a solid.
+__global__ __launch_bounds__(256) void edt_pack(const uint8_t* __restrict__ occ, uint2* __restrict__ bits,
+                                                int nx, int ny, int64_t rows, int words, int R, int wide) {
+    extern __shared__ uint32_t s[];
+    const int64_t row0 = (int64_t)blockIdx.x * R;
+    const int ls = words + 1;                 // odd-even row stride against bank conflicts
+    uint16_t* half = (uint16_t*)s;
+    const int halves = 2 * words;
+    for (int i = threadIdx.x; i < R * halves; i += 256) {
+        const int r = i / halves, h = i - r * halves;
+        const int x0 = h * 16;
+        uint32_t b = 0xffffu;
+        if (row0 + r < rows && x0 < nx) {
+            const uint8_t* o = occ + (row0 + r) * nx + x0;
+            if (wide) {   // nx a multiple of 16 and occ 16-byte aligned
+                const uint4 v = *(const uint4*)o;
+                const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+                b = 0u;
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    // bit 7 of each non-zero byte, gathered into 4 bits
+                    const uint32_t nz = (((w[k] & 0x7f7f7f7fu) + 0x7f7f7f7fu) | w[k]) & 0x80808080u;
+                    b |= (((nz >> 7) * 0x01020408u) >> 24) << (4 * k);
+                }
+            } else {
+                b = 0u;
+#pragma unroll
+                for (int k = 0; k < 16; ++k)
+                    b |= (x0 + k >= nx || o[k] != 0 ? 1u : 0u) << k;
+            }
+        }
+        half[r * 2 * ls + h] = (uint16_t)b;
     }
     __syncthreads();
-    for (int i = threadIdx.x; i < n * T; i += blockDim.x) {
-        const int q = i / T, c = i - (i / T) * T;
-        const int32_t* col = s + c;
-        int32_t best = col[(q + 1) * T];
-        for (int d = 1; d * d < best; ++d) {
-            const int32_t d2 = d * d;
-            best = min(best, col[(q + 1 - d) * T] + d2);
-            best = min(best, col[(q + 1 + d) * T] + d2);
+    for (int i = threadIdx.x; i < R * words; i += 256) {
+        const int w = i / R, r = i - w * R;
+        if (row0 + r >= rows) continue;
+        const uint32_t* line = s + r * ls;
+        int k = w - 1;
+        while (k >= 0 && line[k] == 0u) --k;
+        const int left = k < 0 ? 32 * w + 1 : 32 * w - (32 * k + 31 - __builtin_clz(line[k]));
+        k = w + 1;
+        while (k < words && line[k] == 0u) ++k;
+        // past the last word everything is padding; so is its tail
+        const int right = k >= words ? 32 * words - (32 * w + 31) : 32 * k + __builtin_ctz(line[k]) - (32 * w + 31);
+        const int64_t row = row0 + r, z = row / ny, y = row - z * ny;
+        bits[(z * words + w) * ny + y] = make_uint2(line[w], (uint32_t)left | ((uint32_t)right << 16));
+    }
+}
+
+// Zeros above the top set bit / below the bottom one; no set bit: 2^32 - 1.
+__device__ __forceinline__ uint32_t top_zeros(uint32_t v) { return v ? (uint32_t)__builtin_clz(v) : 0xffffffffu; }
+__device__ __forceinline__ uint32_t low_zeros(uint32_t v) { return v ? (uint32_t)__builtin_ctz(v) : 0xffffffffu; }
+
+// Distance along x of voxel i (0..31) of a packed word to the nearest solid.
+__device__ __forceinline__ uint32_t row_distance(uint2 b, int i) {
+    const uint32_t left = (uint32_t)i + (b.y & 0xffffu), right = (uint32_t)(31 - i) + (b.y >> 16);
+    return min(min(top_zeros(b.x << (31 - i)), low_zeros(b.x >> i)), min(left, right));
+}
+
+// sqrt(x) rounded to nearest, for x >= 2^-60 or 0 of the normal range: the
+// hardware root is within one ulp, and of the three candidates the one whose
+// products with the root bracket x is the rounded one (Markstein's test).
+// For an x that fp32 holds exactly this is the fp64 root rounded to fp32
+// (double rounding is harmless for a root: 53 >= 2*24 + 2 bits).
+__device__ __forceinline__ float sqrt_rn(float x) {
+    float r = __builtin_amdgcn_sqrtf(x);
+    const float lo = __uint_as_float(__float_as_uint(r) - 1u), hi = __uint_as_float(__float_as_uint(r) + 1u);
+    const float below = __builtin_fmaf(-lo, r, x), above = __builtin_fmaf(-hi, r, x);
+    r = below <= 0.0f ? lo : r;
+    return above > 0.0f ? hi : r;
+}
+
+// The same rounded once to fp16 (results of at least 2^-14, or 0): the root
+// lies in the fp16 interval of the hardware's, or an ulp beside one of its
+// ends, so comparing x with the square of the interval's midpoint rounds it.
+__device__ __forceinline__ __half sqrt_rn_f16(float x) {
+    const uint32_t lo = __float_as_uint(__builtin_amdgcn_sqrtf(x)) & ~0x1fffu;
+    const float mid = __uint_as_float(lo | 0x1000u);
+    const float rem = __builtin_fmaf(-mid, mid, x);
+    const bool up = rem > 0.0f || (rem == 0.0f && (lo & 0x2000u) != 0u);
+    return __float2half_rn(__uint_as_float(up ? lo + 0x2000u : lo));
+}
+
+struct PassArgs {
+    const uint2* bits;     // y pass: packed occupancy
+    void* plane;           // squared distances over x and y, pitch voxels a row
+    int pitch;
+    void* out;             // y pass: the plane; z pass: the distances
+    int nx, ny, nz, words;
+    int n, blks;           // line length and its 16-output blocks
+    int tiles;             // tiles along x
+    int64_t blocks;
+    double cell2;
+    float cell2f;          // cell2 in fp32 (where D * cell2 is exact there)
+    int wide;              // z pass: two voxels a store (a row holds a whole number of pairs)
+};
+
+// Row of a tile in LDS: a row's gap after each block of rows, so that the
+// blocks a wave works on lie on different banks.
+template <int TW>
+__device__ __forceinline__ int tile_row(int row) {
+    return (row + row / kBlk) * TW;
+}
+
+// What a pass writes: the plane of squares (y pass), or the distances.
+enum { kPlane, kF32, kF16 };
+
+// The distance of a squared one: fp32 or fp16, rounded once from sqrt(d * cell2).
+template <typename O, bool EXACT>
+__device__ __forceinline__ O distance(const PassArgs& a, uint32_t d) {
+    if constexpr (std::is_same<O, float>::value) {
+        if constexpr (EXACT) return sqrt_rn((float)d * a.cell2f);
+        else return (float)sqrt((double)d * a.cell2);
+    } else {
+        if constexpr (EXACT) return sqrt_rn_f16((float)d * a.cell2f);
+        else return f64_to_f16_rne(sqrt((double)d * a.cell2));
+    }
+}
+
+template <typename V, typename O, bool EXACT>
+__device__ __forceinline__ void put_distances(const PassArgs& a, O* o, V v, int x) {
+    const O d0 = distance<O, EXACT>(a, Word<V>::get(v, 0));
+    if constexpr (Word<V>::kVox == 2) {
+        const O d1 = distance<O, EXACT>(a, Word<V>::get(v, 1));
+        struct alignas(2 * sizeof(O)) Two { O a, b; };
+        if (a.wide) *(Two*)o = Two{d0, d1};
+        else {
+            o[0] = d0;
+            if (x + 1 < a.nx) o[1] = d1;
         }
-        const int64_t b = line_base(c);
-        if (b < 0) continue;
-        const int64_t o = b + (int64_t)q * stride;
-        if constexpr (!LAST) {
-            out[o] = best;
-        } else {
-            const double dist = sqrt((double)best * cell2);
-            if (fout) fout[o] = (float)dist;
-            else hout[o] = f64_to_f16_rne(dist);
+    } else {
+        o[0] = d0;
+    }
+}
+
+template <typename V, int TW, int OUT, bool EXACT>
+__global__ __launch_bounds__(OUT == kPlane ? kThreadsY : kThreadsZ) void edt_tile(PassArgs a) {
+    constexpr bool Z = OUT != kPlane;
+    using W = Word<V>;
+    using P = typename W::Plane;
+    using C = Cell<V, Z>;
+    using T = typename C::T;
+    extern __shared__ uint32_t smem[];
+    T* s = (T*)smem;                                                  // the tile's lines
+    T* cmin = s + (size_t)tile_row<TW>(a.blks * kBlk);                // smallest of each chunk
+    const int64_t tile = xcd_tile(blockIdx.x, a.blocks);
+    const int outer = (int)(tile / a.tiles);             // z (y pass) or y (z pass)
+    const int xt = (int)(tile - (int64_t)outer * a.tiles) * TW * W::kVox;
+    const int n = a.n;
+
+    // a thread keeps its column: the workgroup is a multiple of TW wide
+    const int col = threadIdx.x % TW, x = xt + col * W::kVox;
+    const int row0 = threadIdx.x / TW, rows = blockDim.x / TW;
+    if constexpr (Z) {
+        const P* p = (const P*)a.plane + (int64_t)outer * a.pitch + x;
+        const int64_t step = (int64_t)a.ny * a.pitch;
+        for (int row = row0; row < a.blks * kBlk; row += rows)
+            s[tile_row<TW>(row) + col] = row < n && x < a.nx ? C::shut(*(const V*)(p + row * step)) : C::shut(C::far());
+    } else {
+        const uint2* p = a.bits + ((int64_t)outer * a.words + (x >> 5)) * n;
+        const int i = x & 31;
+        for (int row = row0; row < a.blks * kBlk; row += rows) {
+            V v = C::far();
+            if (row < n && x < a.nx) {
+                const uint2 b = p[row];
+                const uint32_t g0 = row_distance(b, i);
+                if constexpr (W::kVox == 2) {
+                    const uint32_t g1 = row_distance(b, i + 1);
+                    v = u16x2{(unsigned short)min(g0, 255u), (unsigned short)min(g1, 255u)};
+                } else {
+                    v = g0 * g0;
+                }
+            }
+            s[tile_row<TW>(row) + col] = C::shut(v);
+        }
+    }
+    __syncthreads();
+    for (int k = row0; k < a.blks; k += rows) {
+        const T* p = s + tile_row<TW>(k * kBlk) + col;
+        V m = C::open(p[0]);
+#pragma unroll
+        for (int r = 1; r < kBlk; ++r) m = __builtin_elementwise_min(m, C::open(p[r * TW]));
+        cmin[k * TW + col] = C::shut(m);
+    }
+    __syncthreads();
+    if (x >= a.nx) return;
+    const uint32_t cap = Z ? W::kMax : min((uint32_t)(outer + 1) * (uint32_t)(a.nz - outer), W::kMax);   // z_cap
+    for (int blk = row0; blk < a.blks; blk += rows) {
+        const int q0 = blk * kBlk;
+        const T* own = s + tile_row<TW>(q0) + col;
+        V best[kBlk];
+        V most = W::splat(0u);
+#pragma unroll
+        for (int r = 0; r < kBlk; ++r) {
+            // the value above, and the solid rows at -1 and n; rows past the
+            // end take part in nothing
+            const int e = min(q0 + r + 1, n - q0 - r);
+            const uint32_t pad = e > 0 ? min((uint32_t)(e * e), cap) : 0u;
+            best[r] = __builtin_elementwise_min(C::value(C::open(own[r * TW])), W::splat(pad));
+            most = __builtin_elementwise_max(most, best[r]);
+        }
+        // the chunk of rows at p, row j at distance d(j, r) from output r
+        auto take = [&](const T* p, auto square) {
+#pragma unroll
+            for (int j = 0; j < kBlk; ++j) {
+                const V v = C::value(C::open(p[j * TW]));
+#pragma unroll
+                for (int r = 0; r < kBlk; ++r)
+                    best[r] = __builtin_elementwise_min(best[r], W::add(v, square(j, r)));
+            }
+            most = best[0];
+#pragma unroll
+            for (int r = 1; r < kBlk; ++r) most = __builtin_elementwise_max(most, best[r]);
+        };
+        if (W::any_less(C::value(C::open(cmin[blk * TW + col])), most))
+            take(own, [](int j, int r) { return W::splat((uint32_t)((j - r) * (j - r))); });
+        for (int c = 1;; ++c) {
+            const uint32_t near = (uint32_t)(kBlk * (c - 1) + 1);   // of the chunk's nearest row
+            const V near2 = W::splat(min(near * near, W::kMax));
+            const bool go = W::any_less(near2, most);
+            if (!__any(go)) break;
+            const int up = blk + c, down = blk - c;
+            const bool has_up = up < a.blks, has_down = down >= 0;
+            if (!__any(has_up || has_down)) break;
+            // row j is near + j beyond the last output or before the first
+            V sq[2 * kBlk - 1];
+#pragma unroll
+            for (int k = 0; k < 2 * kBlk - 1; ++k)
+                sq[k] = W::splat(min((near + (uint32_t)k) * (near + (uint32_t)k), W::kMax));
+            if (go && has_up && W::any_less(W::add(C::value(C::open(cmin[up * TW + col])), near2), most))
+                take(s + tile_row<TW>(up * kBlk) + col, [&](int j, int r) { return sq[j + kBlk - 1 - r]; });
+            if (go && has_down && W::any_less(W::add(C::value(C::open(cmin[down * TW + col])), near2), most))
+                take(s + tile_row<TW>(down * kBlk) + col, [&](int j, int r) { return sq[kBlk - 1 - j + r]; });
+        }
+        const int64_t step = Z ? (int64_t)a.ny * a.nx : a.pitch;
+        const int64_t first = Z ? ((int64_t)q0 * a.ny + outer) * a.nx + x : ((int64_t)outer * n + q0) * a.pitch + x;
+        using O = typename std::conditional<OUT == kPlane, P, typename std::conditional<OUT == kF32, float, __half>::type>::type;
+        O* o = (O*)a.out + first;
+#pragma unroll
+        for (int r = 0; r < kBlk; ++r) {
+            if (q0 + r < n) {
+                if constexpr (!Z) *(V*)(o + r * step) = best[r];
+                else put_distances<V, O, EXACT>(a, o + r * step, best[r], x);
+            }
         }
     }
 }
 
-// LDS budget of one windowed tile: a few workgroups per CU.
-constexpr int64_t kWindowLds = 40 << 10;
-
-// Which algorithm a pass takes. The envelope walk costs a fixed number of
-// serial steps per line, so it is fast once there are lines enough to keep
-// every SIMD busy; the windowed search costs the distances themselves but
-// spreads them over many waves. Measured (one MI355X): on the 256x256x128
-// ramp_field occupancy (32,768 y lines, 65,536 z lines) the windowed passes
-// take 105 + 66 us against 514 + 243 us; on the 1024x1024x256 winding_track
-// occupancy (262,144 y lines, 1,048,576 z lines; large open spaces) the
-// envelope takes 5.7 + 2.8 ms against 9.4 + 3.8 ms. The windowed search
-// runs while a pass has fewer lines than two waves per SIMD of envelope
-// threads: 512 lines per CU.
-constexpr int64_t kEnvelopeLinesPerCU = 512;
-
-// Tile shape (tx, ty) of a windowed pass over `lines` lines of length n, or
-// (0, 0) for the envelope kernels: when the lines are many enough, or when
-// even four lines do not fit the LDS budget.
-void window_tile(int n, int64_t lines, int cus, bool z_pass, int* tx, int* ty) {
-    static const int shapes[][2] = {{16, 2}, {16, 1}, {8, 1}, {4, 1}};
-    *tx = *ty = 0;
-    if (cus > 0 && lines >= kEnvelopeLinesPerCU * cus) return;
-    for (const auto& sh : shapes) {
-        if (!z_pass && sh[1] != 1) continue;
-        if ((int64_t)(n + 2) * sh[0] * sh[1] * (int64_t)sizeof(int32_t) <= kWindowLds) {
-            *tx = sh[0];
-            *ty = sh[1];
-            return;
+// Words a tile is wide for lines of n, and its LDS bytes; 0 where even the
+// narrowest does not fit the workgroup's LDS.
+int tile_words(int n, int cell_bytes, int64_t lds_limit, size_t* lds) {
+    const int64_t blks = (n + kBlk - 1) / kBlk;
+    for (int tw : {32, 16, 8}) {
+        const int64_t bytes = blks * (kBlk + 2) * tw * cell_bytes;   // rows, gap and minimum
+        if (bytes <= lds_limit) {
+            *lds = (size_t)bytes;
+            return tw;
         }
     }
+    return 0;
+}
+
+template <typename V, int OUT, bool EXACT>
+hipError_t launch_tile(PassArgs a, int tw, size_t lds, int outer, hipStream_t st) {
+    a.blks = (a.n + kBlk - 1) / kBlk;
+    const int vox = tw * Word<V>::kVox;
+    a.tiles = (a.nx + vox - 1) / vox;
+    a.blocks = (int64_t)a.tiles * outer;
+    auto* k = tw == 32 ? edt_tile<V, 32, OUT, EXACT> : tw == 16 ? edt_tile<V, 16, OUT, EXACT> : edt_tile<V, 8, OUT, EXACT>;
+    if (lds > (64 << 10)) {
+        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(k),
+                                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        if (e != hipSuccess) return e;
+    }
+    const int items = a.blks * tw;   // one kBlk-output search each
+    const int most = OUT == kPlane ? kThreadsY : kThreadsZ;
+    const int threads = items >= most ? most : (items + 63) & ~63;
+    k<<<(unsigned)a.blocks, threads, lds, st>>>(a);
+    return hipGetLastError();
+}
+
+template <typename V>
+hipError_t launch_z(const PassArgs& a, bool f32, bool exact, int tw, size_t lds, hipStream_t st) {
+    if (f32) return exact ? launch_tile<V, kF32, true>(a, tw, lds, a.ny, st) : launch_tile<V, kF32, false>(a, tw, lds, a.ny, st);
+    return exact ? launch_tile<V, kF16, true>(a, tw, lds, a.ny, st) : launch_tile<V, kF16, false>(a, tw, lds, a.ny, st);
+}
+
+// Bytes hold every distance along x that can matter (255^2 >= z_cap), and 16
+// bits every square, up to this nz: floor((nz + 1)^2 / 4) <= 65025.
+constexpr int kPackedMaxNz = 509;
+
+// Whether D * cell2 is exact in fp32 for every squared distance D a grid can
+// hold (the padding bounds D by ((n + 1) / 2)^2 along the shortest axis).
+bool exact_in_f32(double cell2, int nx, int ny, int nz) {
+    const int64_t n = nx < ny ? (nx < nz ? nx : nz) : (ny < nz ? ny : nz);
+    const int64_t most = ((n + 1) / 2) * ((n + 1) / 2);
+    int e = 0;
+    double m = frexp(cell2, &e);
+    int bits = 0;
+    while (bits < 54 && m != floor(m)) {
+        m *= 2.0;
+        ++bits;
+    }
+    return (double)most * m < 16777216.0 && cell2 >= 0x1p-28 && cell2 * (double)most < 0x1p100;
 }
 
 // Two int32 planes of the grid, then (8-byte aligned) the uint64 envelope
@@ -369,37 +681,59 @@ SDFR_API int32_t sdfr_edt(const uint8_t* occ, int32_t nx, int32_t ny, int32_t nz
                      (long long)workspace_size);
     if (((uintptr_t)workspace & 7u) != 0) return efail(-2, "sdfr_edt: workspace must be 8-byte aligned");
     const int64_t vox = (int64_t)nx * ny * nz;
-    int32_t* a = (int32_t*)workspace;
-    int32_t* b = a + vox;
-    uint64_t* v = (uint64_t*)((char*)workspace + edt_env_offset(nx, ny, nz));
     hipStream_t st = (hipStream_t)stream;
     const double cell2 = (double)cell * (double)cell;
     const int64_t rows = (int64_t)nz * ny, cols = (int64_t)nz * nx, lines = (int64_t)ny * nx;
     float* fout = out_dtype == SDFR_F32 ? (float*)out : nullptr;
     __half* hout = out_dtype == SDFR_F16 ? (__half*)out : nullptr;
-    edt_rows<<<(int)((rows + 3) / 4), 256, 0, st>>>(occ, a, nx, rows);
-    int dev = 0, cus = 0;
+    int dev = 0, lds_limit = 0;
     if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
-        cus = 0;   // unknown: the windowed passes wherever they fit
-    int tx, ty;
-    window_tile(ny, cols, cus, false, &tx, &ty);
-    if (tx) {
-        const dim3 grid((unsigned)((nx + tx - 1) / tx), (unsigned)nz);
-        edt_window<1, false><<<grid, 256, (size_t)(ny + 2) * tx * ty * sizeof(int32_t), st>>>(
-            a, b, nullptr, nullptr, nx, ny, nz, tx, ty, 0.0);
-    } else {
-        edt_cols<<<(int)((cols + 255) / 256), 256, 0, st>>>(a, b, v, nx, ny, nz);
+        hipDeviceGetAttribute(&lds_limit, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess)
+        lds_limit = 64 << 10;
+    const bool packed = nz <= kPackedMaxNz;
+    size_t lds_y = 0, lds_z = 0;
+    const int tw_y = tile_words(ny, packed ? 2 : 4, lds_limit, &lds_y), tw_z = tile_words(nz, 4, lds_limit, &lds_z);
+    if (tw_y && tw_z) {
+        // the bits, then the plane of squares (edt_scratch_bytes holds both)
+        PassArgs p;
+        memset(&p, 0, sizeof p);
+        p.words = (nx + 31) / 32;
+        p.bits = (const uint2*)workspace;
+        p.plane = (char*)workspace + rows * p.words * (int64_t)sizeof(uint2);
+        p.pitch = packed ? (nx + 1) & ~1 : nx;
+        p.nx = nx;
+        p.ny = ny;
+        p.nz = nz;
+        p.cell2 = cell2;
+        p.cell2f = (float)cell2;
+        const bool exact = exact_in_f32(cell2, nx, ny, nz);
+        p.wide = nx % 2 == 0 && ((uintptr_t)out & (fout ? 7u : 3u)) == 0;
+        int R = 512 / p.words;
+        R = R < 1 ? 1 : R > 32 ? 32 : R;
+        const int wide_in = nx % 16 == 0 && ((uintptr_t)occ & 15u) == 0;
+        edt_pack<<<(unsigned)((rows + R - 1) / R), 256, (size_t)R * (p.words + 1) * 4, st>>>(
+            occ, (uint2*)workspace, nx, ny, rows, p.words, R, wide_in);
+        hipError_t e = hipGetLastError();
+        p.n = ny;
+        p.out = p.plane;
+        if (e == hipSuccess)
+            e = packed ? launch_tile<u16x2, kPlane, true>(p, tw_y, lds_y, nz, st)
+                       : launch_tile<uint32_t, kPlane, true>(p, tw_y, lds_y, nz, st);
+        p.n = nz;
+        p.out = out;
+        if (e == hipSuccess)
+            e = packed ? launch_z<u16x2>(p, fout != nullptr, exact, tw_z, lds_z, st)
+                       : launch_z<uint32_t>(p, fout != nullptr, exact, tw_z, lds_z, st);
+        if (e != hipSuccess) return efail(-4, "sdfr_edt: launch failed: %s", hipGetErrorString(e));
+        return 0;
     }
-    window_tile(nz, lines, cus, true, &tx, &ty);
-    if (tx) {
-        const dim3 grid((unsigned)((nx + tx - 1) / tx), (unsigned)((ny + ty - 1) / ty));
-        edt_window<2, true><<<grid, 256, (size_t)(nz + 2) * tx * ty * sizeof(int32_t), st>>>(
-            b, nullptr, fout, hout, nx, ny, nz, tx, ty, cell2);
-    } else {
-        edt_slabs<<<(int)((lines + 255) / 256), 256, 0, st>>>(b, v, fout, hout, nx, ny, nz,
-                                                              cell2);
-    }
+    // a line too long for LDS: the envelope walk
+    int32_t* a = (int32_t*)workspace;
+    int32_t* b = a + vox;
+    uint64_t* v = (uint64_t*)((char*)workspace + edt_env_offset(nx, ny, nz));
+    edt_rows<<<(int)((rows + 3) / 4), 256, 0, st>>>(occ, a, nx, rows);
+    edt_cols<<<(int)((cols + 255) / 256), 256, 0, st>>>(a, b, v, nx, ny, nz);
+    edt_slabs<<<(int)((lines + 255) / 256), 256, 0, st>>>(b, v, fout, hout, nx, ny, nz, cell2);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return efail(-4, "sdfr_edt: launch failed: %s", hipGetErrorString(e));
     return 0;

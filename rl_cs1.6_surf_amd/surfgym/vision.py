@@ -246,7 +246,12 @@ def sdf_from_occupancy(occ, cell: float, device="cuda", dtype=None) -> torch.Ten
     o = torch.as_tensor(np.asarray(occ) if not torch.is_tensor(occ) else occ)
     if o.dim() != 3:
         raise ValueError(f"occupancy must be [nz, ny, nx], got shape {tuple(o.shape)}")
-    o = (o != 0).to(device=device, dtype=torch.uint8).contiguous()
+    # the bake takes any non-zero byte as solid: uint8 and bool grids on its
+    # device are read as they are
+    if o.device.type == device.type and o.dtype in (torch.uint8, torch.bool):
+        o = o.to(device).contiguous().view(torch.uint8)
+    else:
+        o = (o != 0).to(device=device, dtype=torch.uint8).contiguous()
     nz, ny, nx = (int(v) for v in o.shape)
     if dtype is None:
         dtype = torch.float16 if o.numel() > 100e6 else torch.float32
