@@ -17,9 +17,9 @@
 // therefore relaxes in the order that suits the GPU instead of the
 // reference's whole-grid Jacobi sweeps (one voxel of progress per sweep):
 //
-//   * 8x8x8 tiles, one 512-thread block per tile visit, are loaded with a
-//     one-voxel halo into LDS and relaxed there (Gauss-Seidel, in place)
-//     until the tile is stable — a visit carries a front across a tile;
+//   * 8x8x8 tiles, one wave per tile visit, are loaded with a one-voxel halo
+//     into LDS and relaxed there until the tile is stable — a visit carries a
+//     front across a tile;
 //   * a tile writes back only the voxels it lowered, in place, and queues
 //     the neighbour tiles whose halo holds one of them (a tile is stable
 //     against its halo after a visit, so nothing else needs revisiting);
@@ -56,12 +56,20 @@ __attribute__((format(printf, 2, 3))) int32_t gfail(int32_t code, const char* fm
 
 constexpr int kT = 8;                    // tile edge (voxels)
 constexpr int kH = kT + 2;               // tile edge with halo
-constexpr int kHalo = kH * kH * kH;      // 1000 LDS floats
-constexpr int kThreads = kT * kT * kT;   // one thread per tile voxel
+// LDS floats per column (8 and a gap) and per row of columns: 16-byte reads of
+// 8 lanes along x fall 12 words apart, and 32 mod 64 from the next row's, so
+// the 16 lanes of two rows read all 64 banks once.
+constexpr int kCol = 12, kRow = 160;
+constexpr int kTileLds = kH * kRow + 2 * kH * kH;
+constexpr int kWaves = 4;                // tiles a block visits at once, one a wave
+constexpr int kThreads = 64 * kWaves;
 constexpr int kMaxLocal = 96;            // local sweeps per visit; the tile is requeued if hit
 constexpr int kSweepChunk = 32;          // sweeps launched between host checks
+constexpr int64_t kPartMinTiles = 4096;  // grids of fewer tiles keep one queue
+constexpr int kPartPitch = 32;           // words between the counts of 8 queues: a line each
 
-// control words after the queues (uint32)
+// control words after the queues (uint32); the three counts are here while
+// there is one queue, else in lines of their own (part_of)
 enum { kCount0 = 0, kCount1 = 1, kCount2 = 2, kSeeds = 3, kReach = 4, kLastBusy = 5, kVisitsLo = 6,
        kVisitsHi = 7, kCtl = 8 };
 
@@ -69,7 +77,10 @@ struct GoalArgs {
     const uint8_t* occ;
     float* d;
     uint32_t* mark;       // [tiles] last sweep the tile was queued for
-    uint32_t* queues;     // [3][tiles]
+    uint32_t* queues;     // [2][parts][part_cap], sweep k reads [k & 1]
+    uint32_t* counts;     // [3][parts], part_pitch words apart: sweep k's is [k % 3]
+    int parts;            // queues a sweep's tiles are split into: 8, one per XCD, or 1
+    uint32_t part_cap, part_pitch;
     uint32_t* ctl;        // [kCtl]
     int nx, ny, nz;
     int tx, ty, tz;       // tiles per axis
@@ -77,141 +88,267 @@ struct GoalArgs {
     float w1, w2, w3;     // edge weights for |o|^2 = 1, 2, 3
 };
 
+// Which of 8 queues a tile goes to. A tile's rows (and halo) use 40 of each
+// 128-byte line they touch, so tiles that share lines are kept in one queue,
+// whose sweep blocks run on one XCD (block b on XCD b % 8) and share its L2:
+// blocks of 4 x 2 x 2 tiles, dealt out in order over rows made odd in length,
+// so that neighbours along every axis go to different queues.
+__device__ __forceinline__ uint32_t part_of(const GoalArgs& a, int tx, int ty, int tz) {
+    if (a.parts == 1) return 0u;
+    const uint32_t sx = (uint32_t)((a.tx + 3) >> 2) | 1u, sy = (uint32_t)((a.ty + 1) >> 1);
+    return (((uint32_t)(tz >> 1) * sy + (uint32_t)(ty >> 1)) * sx + (uint32_t)(tx >> 2)) & 7u;
+}
+
+__device__ __forceinline__ uint32_t* count_of(const GoalArgs& a, uint32_t k, uint32_t part) {
+    return a.counts + ((k % 3u) * (uint32_t)a.parts + part) * a.part_pitch;
+}
+
+__device__ __forceinline__ uint32_t* queue_of(const GoalArgs& a, uint32_t k, uint32_t part) {
+    return a.queues + ((size_t)(k & 1u) * a.parts + part) * a.part_cap;
+}
+
 // d = +inf everywhere, 0 on the free voxels of the seed box; the tiles that
-// hold a seed or touch one through their halo form the first queue.
+// hold a seed or touch one through their halo form the first queue. Four
+// distances per store (the distances start the workspace, which the bake
+// requires 64-byte aligned).
 __global__ __launch_bounds__(256) void goal_init(GoalArgs a, int lx, int ly, int lz, int hx, int hy,
                                                  int hz, int tlx, int tly, int tlz, int thx, int thy,
                                                  int thz) {
-    const int64_t vox = (int64_t)a.nx * a.ny * a.nz;
+    const int64_t vox = (int64_t)a.nx * a.ny * a.nz, n4 = (vox + 3) >> 2;
+    const int64_t step = (int64_t)gridDim.x * blockDim.x, first = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     uint32_t seeds = 0;
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < vox;
-         i += (int64_t)gridDim.x * blockDim.x) {
-        const int x = (int)(i % a.nx);
-        const int64_t r = i / a.nx;
-        const int y = (int)(r % a.ny), z = (int)(r / a.ny);
+    auto value = [&](int64_t i, int x, int y, int z) {
         const bool seed = x >= lx && x <= hx && y >= ly && y <= hy && z >= lz && z <= hz && !a.occ[i];
-        a.d[i] = seed ? 0.0f : INFINITY;
         seeds += seed;
+        return seed ? 0.0f : INFINITY;
+    };
+    for (int64_t i = first; i < n4; i += step) {
+        const int64_t v0 = i << 2, r = v0 / a.nx;
+        int x = (int)(v0 - r * a.nx), y = (int)(r % a.ny), z = (int)(r / a.ny);
+        float v[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            v[j] = v0 + j < vox ? value(v0 + j, x, y, z) : 0.0f;
+            if (++x == a.nx) {
+                x = 0;
+                if (++y == a.ny) {
+                    y = 0;
+                    ++z;
+                }
+            }
+        }
+        if (v0 + 3 < vox) *(float4*)(a.d + v0) = make_float4(v[0], v[1], v[2], v[3]);
+        else
+            for (int j = 0; v0 + j < vox; ++j) a.d[v0 + j] = v[j];
     }
-    const int bnx = thx - tlx + 1, bny = thy - tly + 1;
-    for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < a.tiles;
-         t += (int64_t)gridDim.x * blockDim.x) {
+    for (int64_t t = first; t < a.tiles; t += step) {
         const int tx = (int)(t % a.tx);
         const int64_t r = t / a.tx;
         const int ty = (int)(r % a.ty), tz = (int)(r / a.ty);
         const bool in = tx >= tlx && tx <= thx && ty >= tly && ty <= thy && tz >= tlz && tz <= thz;
         a.mark[t] = in ? 1u : 0u;
-        if (in) a.queues[1 * a.tiles + ((tz - tlz) * bny + (ty - tly)) * bnx + (tx - tlx)] = (uint32_t)t;
+        if (in) {
+            const uint32_t part = part_of(a, tx, ty, tz);
+            queue_of(a, 1u, part)[atomicAdd(count_of(a, 1u, part), 1u)] = (uint32_t)t;
+        }
     }
     for (int off = 32; off > 0; off >>= 1) seeds += __shfl_down(seeds, off);
     if ((threadIdx.x & 63) == 0 && seeds) atomicAdd(&a.ctl[kSeeds], seeds);
 }
 
-__device__ __forceinline__ float relax_voxel(const float* s, int c, float m, float w1, float w2,
-                                             float w3) {
-#pragma unroll
-    for (int oz = -1; oz <= 1; ++oz)
-#pragma unroll
-        for (int oy = -1; oy <= 1; ++oy)
-#pragma unroll
-            for (int ox = -1; ox <= 1; ++ox) {
-                const int q = oz * oz + oy * oy + ox * ox;
-                if (q == 0) continue;
-                const float w = q == 1 ? w1 : (q == 2 ? w2 : w3);
-                m = fminf(m, s[c + (oz * kH + oy) * kH + ox] + w);
-            }
-    return m;
+// The smaller of two distances: of non-negative floats (+inf among them) as
+// their bit patterns order, which spares the compiler the quieting of NaNs.
+__device__ __forceinline__ float least(float a, float b) {
+    return __uint_as_float(min(__float_as_uint(a), __float_as_uint(b)));
 }
 
-// Sweep k: visit every tile of queue k%3, fill queue (k+1)%3, clear the
-// count of queue (k+2)%3 (consumed by sweep k-1, filled by sweep k+1).
+// Lane masks of a tile's columns (lane = 8 * y + x): those on its low / any /
+// high side along x and along y.
+__device__ __forceinline__ uint64_t side_x(int d) {
+    return d < 0 ? 0x0101010101010101ull : d > 0 ? 0x8080808080808080ull : ~0ull;
+}
+__device__ __forceinline__ uint64_t side_y(int d) {
+    return d < 0 ? 0xffull : d > 0 ? 0xffull << 56 : ~0ull;
+}
+
+// Orders a wave's LDS writes before its later reads (one wave owns the tile,
+// and its LDS operations execute in order).
+__device__ __forceinline__ void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Sweep k: visit every tile queued for it, queue tiles for sweep k + 1, clear
+// the counts of sweep k + 2 (those of sweep k - 1).
+//
+// One wave visits one tile, a lane per (x, y) column with its 8 voxels in
+// registers. The 10 x 10 columns with the halo lie in LDS, z fastest, so a
+// relaxation reads each of a column's 8 neighbour columns with two 16-byte
+// loads. x -> fl(x + w) is monotone, so fl(min(a, b) + w) = min(fl(a + w),
+// fl(b + w)): the four face columns and the four edge columns are reduced
+// before their weights are added (2 wide LDS reads and ~17 vector
+// instructions a voxel instead of 26 and 52). Up and down its own column a
+// lane relaxes in order, so a value crosses the tile along z in one pass.
+//
+// What bounds it: in the ~20 long sweeps of a bake the lines the tiles read
+// (240 misses a visit with tiles dealt to any XCD, 3.6 TB/s; queues by XCD
+// took the longest from 39 to 27 us), in the ~40 short ones the chain of
+// round trips to memory of one visit (queue, tile, mark, slot: 8-11 us).
+// 256x256x128 voxels, 58 sweeps: 29 us a sweep with a block of 512 threads
+// and 26 LDS reads a voxel, 18 with a wave a tile, 16 with the columns loaded
+// straight to their lanes, 13 with a queue per XCD. Also measured: flags per
+// tile instead of queues (no claims, but a static deal of tiles to waves: 28
+// us), reading a mark before its atomic (+2 us), no order along z (+2 us),
+// queueing only tiles whose halo copy would fall (20% fewer visits, each 3 us
+// longer).
 __global__ __launch_bounds__(kThreads) void goal_sweep(GoalArgs a, uint32_t k) {
-    __shared__ float s[kHalo];
-    __shared__ uint32_t s_push;
-    const uint32_t qin = k % 3u, qout = (k + 1u) % 3u;
-    const uint32_t n = a.ctl[qin];
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        a.ctl[(k + 2u) % 3u] = 0u;
+    __shared__ __align__(16) float s_all[kWaves][kTileLds];
+    const uint32_t part = blockIdx.x % (uint32_t)a.parts, block = blockIdx.x / (uint32_t)a.parts;
+    const uint32_t blocks = gridDim.x / (uint32_t)a.parts;   // of this queue
+    const uint32_t* qi = queue_of(a, k, part);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    // consecutive tiles go to different blocks: a short queue spreads over the
+    // GPU. The first entry is read with the length, not after it (an entry
+    // past the queue's end is not used).
+    uint32_t e = (uint32_t)wave * blocks + block;
+    uint32_t tile_v = e < a.part_cap ? qi[e] : 0u;
+    const uint32_t n = *count_of(a, k, part);
+    if (block == 0 && threadIdx.x == 0) {
+        *count_of(a, k + 2u, part) = 0u;
         if (n) {
             a.ctl[kLastBusy] = k;
             atomicAdd((unsigned long long*)&a.ctl[kVisitsLo], (unsigned long long)n);
         }
     }
-    const uint32_t* qi = a.queues + (size_t)qin * a.tiles;
-    uint32_t* qo = a.queues + (size_t)qout * a.tiles;
-    const int tid = threadIdx.x;
-    const int lx = tid & 7, ly = (tid >> 3) & 7, lz = tid >> 6;
-    const int c = ((lz + 1) * kH + (ly + 1)) * kH + (lx + 1);
-    for (uint32_t e = blockIdx.x; e < n; e += gridDim.x) {
-        const uint32_t tile = qi[e];
+    const int lx = lane & 7, ly = lane >> 3;
+    float* s = s_all[wave];
+    float* zlo = s + kH * kRow;         // the halo planes below and above
+    float* zhi = zlo + kH * kH;
+    const int c = (ly + 1) * kH + (lx + 1);
+    float* own = s + (ly + 1) * kRow + (lx + 1) * kCol;
+    const float w1 = a.w1, w2 = a.w2, w3 = a.w3;
+    // lanes 0..35 also load a halo column each: the sides x = -1, x = 8,
+    // y = -1, y = 8 (8 lanes each), then the corners
+    const int side = lane >> 3, at = (lane & 7) + 1;
+    const int rx = side == 0 ? 0 : side == 1 ? kH - 1 : side > 3 ? (lane & 1) * (kH - 1) : at;
+    const int ry = side == 2 ? 0 : side == 3 ? kH - 1 : side > 3 ? ((lane >> 1) & 1) * (kH - 1) : at;
+    float* ring = s + ry * kRow + rx * kCol;
+    for (; e < n; e += blocks * kWaves, tile_v = e < n ? qi[e] : 0u) {
+        const uint32_t tile = __builtin_amdgcn_readfirstlane(tile_v);
         const int tx = (int)(tile % (uint32_t)a.tx);
         const uint32_t r = tile / (uint32_t)a.tx;
         const int ty = (int)(r % (uint32_t)a.ty), tz = (int)(r / (uint32_t)a.ty);
-        const int x0 = tx * kT - 1, y0 = ty * kT - 1, z0 = tz * kT - 1;
-        for (int i = tid; i < kHalo; i += kThreads) {
-            const int hx = i % kH, hy = (i / kH) % kH, hz = i / (kH * kH);
-            const int x = x0 + hx, y = y0 + hy, z = z0 + hz;
-            float v = INFINITY;   // outside the grid: never lowers a neighbour
-            if (x >= 0 && y >= 0 && z >= 0 && x < a.nx && y < a.ny && z < a.nz)
-                v = a.d[((int64_t)z * a.ny + y) * a.nx + x];
-            s[i] = v;
+        const int x0 = tx * kT, y0 = ty * kT, z0 = tz * kT;
+        const int x = x0 + lx, y = y0 + ly, xr = x0 + rx - 1, yr = y0 + ry - 1;
+        const bool inside = x < a.nx && y < a.ny;
+        const bool on_ring = lane < 36 && xr >= 0 && yr >= 0 && xr < a.nx && yr < a.ny;
+        const int64_t idx = ((int64_t)z0 * a.ny + y) * a.nx + x, plane = (int64_t)a.ny * a.nx;
+        const int64_t rdx = ((int64_t)z0 * a.ny + yr) * a.nx + xr;
+        // the lane's own column and its halo column, both with the voxels
+        // below and above; outside the grid nothing lowers a neighbour
+        float cv[kH], rv[kH];
+        bool open[kT];
+#pragma unroll
+        for (int z = 0; z < kH; ++z) {
+            const bool in_z = z0 + z - 1 >= 0 && z0 + z - 1 < a.nz;   // uniform
+            cv[z] = rv[z] = INFINITY;
+            if (in_z && inside) cv[z] = a.d[idx + (z - 1) * plane];
+            if (in_z && on_ring) rv[z] = a.d[rdx + (z - 1) * plane];
         }
-        const int x = x0 + 1 + lx, y = y0 + 1 + ly, z = z0 + 1 + lz;
-        const bool inside = x < a.nx && y < a.ny && z < a.nz;
-        const int64_t idx = ((int64_t)z * a.ny + y) * a.nx + x;
-        const bool open = inside && a.occ[idx] == 0;
-        if (tid == 0) s_push = 0u;
-        __syncthreads();
-        const float start = s[c];
-        // Gauss-Seidel in LDS: only this thread writes s[c]; a neighbour read
-        // sees the old or the new value, both path sums. A local sweep in
-        // which no voxel lowered saw a constant tile: the tile is stable.
-        int moving = 1;
-        int it = 0;
-        while (moving && it < kMaxLocal) {
-            int lowered = 0;
-            if (open) {
-                const float cur = s[c];
-                const float m = relax_voxel(s, c, cur, a.w1, a.w2, a.w3);
-                if (m < cur) {
-                    s[c] = m;
-                    lowered = 1;
-                }
+#pragma unroll
+        for (int z = 0; z < kT; ++z) open[z] = inside && z0 + z < a.nz && a.occ[idx + z * plane] == 0;
+        float start[kT], cur[kT];
+#pragma unroll
+        for (int z = 0; z < kT; ++z) start[z] = cur[z] = cv[z + 1];
+        *(float4*)own = make_float4(cv[1], cv[2], cv[3], cv[4]);
+        *(float4*)(own + 4) = make_float4(cv[5], cv[6], cv[7], cv[8]);
+        zlo[c] = cv[0];
+        zhi[c] = cv[kH - 1];
+        if (lane < 36) {
+            *(float4*)ring = make_float4(rv[1], rv[2], rv[3], rv[4]);
+            *(float4*)(ring + 4) = make_float4(rv[5], rv[6], rv[7], rv[8]);
+            zlo[ry * kH + rx] = rv[0];
+            zhi[ry * kH + rx] = rv[kH - 1];
+        }
+        wave_sync();
+        // what the planes below and above give the first and last voxel
+        // (the halo does not change during a visit)
+        auto beside = [&](const float* p) {
+            const float f = least(least(p[c - 1], p[c + 1]), least(p[c - kH], p[c + kH]));
+            const float g = least(least(p[c - kH - 1], p[c - kH + 1]), least(p[c + kH - 1], p[c + kH + 1]));
+            return least(least(f + w2, g + w3), p[c] + w1);
+        };
+        const float below = beside(zlo), above = beside(zhi);
+        // a pass in which no voxel lowered saw a constant tile: it is stable
+        bool moving = true;
+        for (int it = 0; moving && it < kMaxLocal; ++it) {
+            float f[kT], g[kT];
+            auto column = [&](int o, float* m, bool first) {
+                const float4 lo = *(const float4*)(own + o), hi = *(const float4*)(own + o + 4);
+                const float q[kT] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+#pragma unroll
+                for (int z = 0; z < kT; ++z) m[z] = first ? q[z] : least(m[z], q[z]);
+            };
+            column(-kCol, f, true);
+            column(kCol, f, false);
+            column(-kRow, f, false);
+            column(kRow, f, false);
+            column(-kRow - kCol, g, true);
+            column(-kRow + kCol, g, false);
+            column(kRow - kCol, g, false);
+            column(kRow + kCol, g, false);
+            // by the voxels above and below: Q the neighbour columns' share,
+            // and the column's own
+            float q[kT], m[kT];
+#pragma unroll
+            for (int z = 0; z < kT; ++z) q[z] = least(least(f[z] + w2, g[z] + w3), cur[z] + w1);
+#pragma unroll
+            for (int z = 0; z < kT; ++z) {
+                m[z] = least(least(cur[z], least(f[z] + w1, g[z] + w2)),
+                             least(z ? q[z - 1] : below, z < kT - 1 ? q[z + 1] : above));
+                if (z) m[z] = least(m[z], m[z - 1] + w1);
+                m[z] = open[z] ? m[z] : INFINITY;
             }
-            moving = __syncthreads_or(lowered);
-            ++it;
+#pragma unroll
+            for (int z = kT - 2; z >= 0; --z) m[z] = open[z] ? least(m[z], m[z + 1] + w1) : INFINITY;
+            bool lowered = false;
+#pragma unroll
+            for (int z = 0; z < kT; ++z) {
+                lowered |= m[z] < cur[z];
+                cur[z] = m[z];
+            }
+            moving = __any(lowered);
+            if (lowered) {
+                *(float4*)own = make_float4(cur[0], cur[1], cur[2], cur[3]);
+                *(float4*)(own + 4) = make_float4(cur[4], cur[5], cur[6], cur[7]);
+            }
+            wave_sync();
         }
-        const float fin = s[c];
-        uint32_t bits = 0;
-        if (fin < start) {
-            a.d[idx] = fin;
-            // neighbour tiles whose halo holds this voxel: per axis, offset 0
-            // always, -1 on the tile's low face, +1 on its high face
-            const int xs0 = lx == 0 ? -1 : 0, xs1 = lx == kT - 1 ? 1 : 0;
-            const int ys0 = ly == 0 ? -1 : 0, ys1 = ly == kT - 1 ? 1 : 0;
-            const int zs0 = lz == 0 ? -1 : 0, zs1 = lz == kT - 1 ? 1 : 0;
-            for (int dz = zs0; dz <= zs1; ++dz)
-                for (int dy = ys0; dy <= ys1; ++dy)
-                    for (int dx = xs0; dx <= xs1; ++dx)
-                        bits |= 1u << ((dz + 1) * 9 + (dy + 1) * 3 + (dx + 1));
-            bits &= ~(1u << 13);
+        bool any = false;
+#pragma unroll
+        for (int z = 0; z < kT; ++z) {
+            if (cur[z] < start[z]) {
+                a.d[idx + z * plane] = cur[z];
+                any = true;
+            }
         }
-        if (moving && tid == 0) bits |= 1u << 13;   // local cap hit: visit again
-        if (bits) atomicOr(&s_push, bits);
-        __syncthreads();
-        const uint32_t push = s_push;
-        if (tid < 27 && ((push >> tid) & 1u)) {
-            const int dz = tid / 9 - 1, dy = (tid / 3) % 3 - 1, dx = tid % 3 - 1;
+        // neighbour tiles whose halo holds a lowered voxel; lane t < 27 looks
+        // after direction t
+        const uint64_t b0 = __ballot(any), bl = __ballot(cur[0] < start[0]), bh = __ballot(cur[kT - 1] < start[kT - 1]);
+        const int dz = lane / 9 - 1, dy = (lane / 3) % 3 - 1, dx = lane % 3 - 1;
+        bool push = ((dz < 0 ? bl : dz > 0 ? bh : b0) & side_x(dx) & side_y(dy)) != 0;
+        if (lane == 13) push = moving;   // the local cap was hit: visit this one again
+        if (lane < 27 && push) {
             const int ux = tx + dx, uy = ty + dy, uz = tz + dz;
             if (ux >= 0 && uy >= 0 && uz >= 0 && ux < a.tx && uy < a.ty && uz < a.tz) {
                 const uint32_t u = ((uint32_t)uz * (uint32_t)a.ty + (uint32_t)uy) * (uint32_t)a.tx + (uint32_t)ux;
-                if (atomicMax(&a.mark[u], k + 1u) < k + 1u) {
-                    const uint32_t slot = atomicAdd(&a.ctl[qout], 1u);
-                    qo[slot] = u;
+                if (atomicMax(&a.mark[u], k + 1u) <= k) {
+                    const uint32_t to = part_of(a, ux, uy, uz);
+                    queue_of(a, k + 1u, to)[atomicAdd(count_of(a, k + 1u, to), 1u)] = u;
                 }
             }
         }
-        __syncthreads();   // s and s_push are reused by the next visit
     }
 }
 
@@ -220,8 +357,10 @@ __global__ __launch_bounds__(kThreads) void goal_sweep(GoalArgs a, uint32_t k) {
 // which the bake requires 64-byte aligned), the last vox % 4 one at a time;
 // one atomic per block (atomics from every wave to the one word serialise).
 constexpr int kReachBlocks = 512;
-__global__ __launch_bounds__(256) void goal_reach_max(const float* d, int64_t vox, uint32_t* best) {
+__global__ __launch_bounds__(256) void goal_reach_max(GoalArgs a, int64_t vox) {
+    const float* d = a.d;
     __shared__ uint32_t s_m[4];
+
     uint32_t m = 0;
     const int64_t n4 = vox >> 2;
     const float4* d4 = reinterpret_cast<const float4*>(d);
@@ -242,7 +381,7 @@ __global__ __launch_bounds__(256) void goal_reach_max(const float* d, int64_t vo
     __syncthreads();
     if (threadIdx.x == 0) {
         m = max(max(s_m[0], s_m[1]), max(s_m[2], s_m[3]));
-        if (m) atomicMax(best, m);
+        if (m) atomicMax(a.ctl + kReach, m);
     }
 }
 
@@ -250,15 +389,30 @@ __global__ __launch_bounds__(256) void goal_reach_max(const float* d, int64_t vo
 // reference divides a CUDA tensor by a Python scalar, which torch evaluates as
 // d * (1/quant) with the reciprocal rounded to fp32 (identical to d / quant
 // for the power-of-two cells the reference picks), and rounds half to even.
-__global__ __launch_bounds__(256) void goal_quantise(const float* d, int64_t vox, float sentinel,
+// The sentinel is the host's reach_max + 2*cell, from the largest distance
+// goal_reach_max left; a field beyond the uint16 range writes nothing. Four
+// voxels a thread (`wide`: the outputs are aligned for it).
+__global__ __launch_bounds__(256) void goal_quantise(const float* d, int64_t vox, const uint32_t* reach, double cell,
                                                      float inv_quant, float quant, uint16_t* q_out,
-                                                     float* g_out) {
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < vox;
-         i += (int64_t)gridDim.x * blockDim.x) {
-        float v = d[i];
+                                                     float* g_out, int wide) {
+    const double sentinel_d = (double)__uint_as_float(*reach) + 2.0 * cell;
+    if (sentinel_d / (cell / 8.0) > 65535.0) return;
+    const float sentinel = (float)sentinel_d;
+    auto code = [&](float v) {
         if (v == INFINITY) v = sentinel;
-        const float q = fminf(fmaxf(rintf(v * inv_quant), 0.0f), 65535.0f);
-        const uint16_t u = (uint16_t)q;
+        return (uint16_t)fminf(fmaxf(rintf(v * inv_quant), 0.0f), 65535.0f);
+    };
+    const int64_t step = (int64_t)gridDim.x * blockDim.x, first = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t n4 = wide ? vox >> 2 : 0;
+    for (int64_t i = first; i < n4; i += step) {
+        const float4 v = ((const float4*)d)[i];
+        const ushort4 u = make_ushort4(code(v.x), code(v.y), code(v.z), code(v.w));
+        if (q_out) ((ushort4*)q_out)[i] = u;
+        if (g_out)
+            ((float4*)g_out)[i] = make_float4((float)u.x * quant, (float)u.y * quant, (float)u.z * quant, (float)u.w * quant);
+    }
+    for (int64_t i = (n4 << 2) + first; i < vox; i += step) {
+        const uint16_t u = code(d[i]);
         if (q_out) q_out[i] = u;
         if (g_out) g_out[i] = (float)u * quant;
     }
@@ -387,61 +541,72 @@ SDFR_API int32_t sdfr_goal_bake(const uint8_t* occ, int32_t nx, int32_t ny, int3
     g.w1 = (float)((double)cell * sqrt(1.0));
     g.w2 = (float)((double)cell * sqrt(2.0));
     g.w3 = (float)((double)cell * sqrt(3.0));
-    const uint32_t first = (uint32_t)(thi[0] - tlo[0] + 1) * (uint32_t)(thi[1] - tlo[1] + 1) *
-                           (uint32_t)(thi[2] - tlo[2] + 1);
-    uint32_t ctl0[kCtl] = {0, first, 0, 0, 0, 0, 0, 0};
-    hipError_t e = hipMemcpyAsync(g.ctl, ctl0, sizeof ctl0, hipMemcpyHostToDevice, st);
+    // eight queues where the queue space holds them and there are tiles enough
+    // to keep them even, else one; the counts then lie right before the
+    // control words, in the queues' space
+    const int64_t part_cap = (((((int64_t)g.tx + 3) / 4) | 1) * ((g.ty + 1) / 2) * ((g.tz + 1) / 2) + 7) / 8 * 16;
+    const int64_t count_words = 3 * 8 * kPartPitch;
+    g.parts = L.tiles >= kPartMinTiles && 16 * part_cap + count_words <= 3 * (int64_t)L.tiles ? 8 : 1;
+    g.part_cap = g.parts == 8 ? (uint32_t)part_cap : L.tiles;
+    g.part_pitch = g.parts == 8 ? kPartPitch : 1;
+    g.counts = g.parts == 8 ? g.ctl - count_words : g.ctl + kCount0;
+    const int64_t shared = (g.parts == 8 ? count_words : 0) + kCtl;   // words the host reads
+    uint32_t host[3 * 8 * kPartPitch + kCtl];
+    uint32_t* const host_ctl = host + (shared - kCtl);
+    uint32_t* const host_counts = g.parts == 8 ? host : host_ctl + kCount0;
+    memset(host, 0, sizeof host);
+    uint32_t* const dev_words = g.ctl - (shared - kCtl);
+    hipError_t e = hipMemcpyAsync(dev_words, host, shared * 4, hipMemcpyHostToDevice, st);
     if (e != hipSuccess) return gfail(-4, "sdfr_goal_bake: %s", hipGetErrorString(e));
-    int init_blocks = (int)((L.vox + 255) / 256);
-    if (init_blocks > 8192) init_blocks = 8192;
+    const int64_t fours = (L.vox + 1023) / 1024;   // four voxels a thread
+    const int init_blocks = (int)(fours > 8192 ? 8192 : fours);
     goal_init<<<init_blocks, 256, 0, st>>>(g, lo[0], lo[1], lo[2], hi[0], hi[1], hi[2], tlo[0], tlo[1],
                                            tlo[2], thi[0], thi[1], thi[2]);
     int dev = 0, cus = 256;
     if (hipGetDevice(&dev) != hipSuccess ||
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
         cus = 256;
-    const int sweep_blocks = cus * 4;   // 4 x 512 threads fill a CU's wave slots
-    uint32_t host[kCtl];
+    const int sweep_blocks = cus * 5 / 8 * 8 > 0 ? cus * 5 / 8 * 8 : 8;   // 5 a CU fit its registers; a multiple of the queues
     uint32_t k = 1;
     bool done = false;
     while (!done && (int64_t)k <= max_sweeps) {
         for (int j = 0; j < kSweepChunk && (int64_t)k <= max_sweeps; ++j, ++k)
             goal_sweep<<<sweep_blocks, kThreads, 0, st>>>(g, k);
         e = hipGetLastError();
-        if (e == hipSuccess) e = hipMemcpyAsync(host, g.ctl, sizeof host, hipMemcpyDeviceToHost, st);
+        if (e == hipSuccess) e = hipMemcpyAsync(host, dev_words, shared * 4, hipMemcpyDeviceToHost, st);
         if (e == hipSuccess) e = hipStreamSynchronize(st);
         if (e != hipSuccess) return gfail(-4, "sdfr_goal_bake: %s", hipGetErrorString(e));
-        if (host[kSeeds] == 0)
+        if (host_ctl[kSeeds] == 0)
             return gfail(-5, "sdfr_goal_bake: goal zone contains no free voxel");
-        if (host[k % 3u] == 0) done = true;   // k is the next sweep: its queue is empty
+        done = true;   // k is the next sweep: are its queues empty?
+        for (int p = 0; p < g.parts; ++p)
+            if (host_counts[((k % 3u) * g.parts + p) * g.part_pitch]) done = false;
     }
     if (!done) return gfail(-7, "sdfr_goal_bake: not converged after %d sweeps", max_sweeps);
-    goal_reach_max<<<kReachBlocks, 256, 0, st>>>(g.d, L.vox, g.ctl + kReach);
+    goal_reach_max<<<kReachBlocks, 256, 0, st>>>(g, L.vox);
+    const double quant = (double)cell / 8.0;
+    const float quant_f = (float)quant;
+    const float inv_quant = 1.0f / quant_f;
+    const int wide = ((uintptr_t)grid_q & 7u) == 0 && ((uintptr_t)grid & 15u) == 0;
+    goal_quantise<<<init_blocks, 256, 0, st>>>(g.d, L.vox, g.ctl + kReach, (double)cell, inv_quant, quant_f, grid_q,
+                                               grid, wide);
     e = hipGetLastError();
-    if (e == hipSuccess) e = hipMemcpyAsync(host, g.ctl, sizeof host, hipMemcpyDeviceToHost, st);
+    if (e == hipSuccess) e = hipMemcpyAsync(host_ctl, g.ctl, kCtl * 4, hipMemcpyDeviceToHost, st);
     if (e == hipSuccess) e = hipStreamSynchronize(st);
     if (e != hipSuccess) return gfail(-4, "sdfr_goal_bake: %s", hipGetErrorString(e));
     float reach_max;
-    memcpy(&reach_max, &host[kReach], 4);
+    memcpy(&reach_max, &host_ctl[kReach], 4);
     // Python floats: sentinel = reach_max + 2*cell, quant = cell/8; stored fp32
     const double sentinel = (double)reach_max + 2.0 * (double)cell;
-    const double quant = (double)cell / 8.0;
     info->reach_max = reach_max;
     info->sentinel = (float)sentinel;
-    info->quant = (float)quant;
-    info->sweeps = (int32_t)host[kLastBusy];
-    info->n_seed = (int64_t)host[kSeeds];
-    info->tile_visits = (int64_t)host[kVisitsLo] | ((int64_t)host[kVisitsHi] << 32);
+    info->quant = quant_f;
+    info->sweeps = (int32_t)host_ctl[kLastBusy];
+    info->n_seed = (int64_t)host_ctl[kSeeds];
+    info->tile_visits = (int64_t)host_ctl[kVisitsLo] | ((int64_t)host_ctl[kVisitsHi] << 32);
     if (sentinel / quant > 65535.0)
         return gfail(-6, "sdfr_goal_bake: sentinel %.0fu exceeds the uint16 range at quant %gu",
                      sentinel, quant);
-    const float quant_f = (float)quant;
-    const float inv_quant = 1.0f / quant_f;
-    goal_quantise<<<init_blocks, 256, 0, st>>>(g.d, L.vox, (float)sentinel, inv_quant, quant_f, grid_q,
-                                               grid);
-    e = hipGetLastError();
-    if (e == hipSuccess) e = hipStreamSynchronize(st);
-    if (e != hipSuccess) return gfail(-4, "sdfr_goal_bake: %s", hipGetErrorString(e));
     return 0;
 }
 

@@ -237,7 +237,12 @@ def goal_field_from_occupancy(occ, mins, zone, cell: float, device="cuda", *, ke
     o = occ if torch.is_tensor(occ) else torch.from_numpy(np.ascontiguousarray(occ))
     if o.dim() != 3:
         raise ValueError(f"occupancy must be [nz, ny, nx], got shape {tuple(o.shape)}")
-    o = (o != 0).to(device=dev, dtype=torch.uint8).contiguous()
+    # the bake takes any non-zero byte as solid: uint8 and bool grids on its
+    # device are read as they are
+    if o.device == dev and o.dtype in (torch.uint8, torch.bool):
+        o = o.contiguous().view(torch.uint8)
+    else:
+        o = (o != 0).to(device=dev, dtype=torch.uint8).contiguous()
     nz, ny, nx = (int(v) for v in o.shape)
     lo, hi = seed_voxel_box(zone, mins, cell, (nx, ny, nz))
     if np.any(hi < lo):

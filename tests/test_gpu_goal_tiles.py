@@ -1,0 +1,64 @@
+"""The goal-field bake's tiles and queues at their edges, against the oracle's fixpoint bit for
+bit: grids of many tiles (a queue per XCD) whose sides end inside a tile, a thin one whose queue
+space holds a single queue only, one long enough for several rounds of sweeps, and the
+quantisation of voxel counts and outputs that allow no four-voxel stores."""
+from __future__ import annotations
+
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import goal as ogoal
+from surfgym import _sdfr, goalfield
+
+pytestmark = pytest.mark.gpu
+
+
+def _occupancy(shape, seed):
+    rng = np.random.default_rng(seed)
+    occ = (rng.random(shape) < 0.25).astype(np.uint8)
+    occ[shape[0] // 2, : shape[1] - 2] = 1     # a wall to go round
+    return occ
+
+
+@pytest.mark.parametrize("shape", [(129, 131, 135), (128, 130, 136), (521, 523, 5), (3, 1030, 1029), (6, 7, 4099)],
+                         ids=str)
+def test_many_tiles_match_oracle(dev, shape):
+    occ = _occupancy(shape, sum(shape))
+    nz, ny, nx = shape
+    occ[0:2, 0:2, 0:2] = 0
+    zone = {"mins": [0.5, 0.5, 0.5], "maxs": [9.0, 9.0, 9.0]}
+    lo, hi = goalfield.seed_voxel_box(zone, np.zeros(3), 8.0, (nx, ny, nz))
+    print(f"case goal tiles {shape}", flush=True)
+    ref = ogoal.bake(occ, 8.0, lo, hi)
+    for form in (occ, torch.as_tensor(occ, device=dev), torch.as_tensor(occ * 3, device=dev) != 0):
+        field = goalfield.goal_field_from_occupancy(form, np.zeros(3), zone, 8.0, device=dev)
+        assert np.array_equal(field.grid_q.cpu().numpy().view(np.uint16), ref["grid_q"])
+        assert np.array_equal(field.grid.cpu().numpy(), ref["grid"])
+        assert np.float32(field.reach_max) == ref["reach_max"]
+
+
+@pytest.mark.parametrize("shift", [0, 1])
+def test_quantised_outputs_at_any_alignment(dev, shift):
+    """Through the C ABI: an odd voxel count, outputs `shift` elements into their buffers."""
+    shape = (9, 11, 13)
+    occ = torch.as_tensor(_occupancy(shape, 3), device=dev)
+    occ[0, 0, 0] = 0
+    n = occ.numel()
+    lib = _sdfr.load()
+    lo = (ctypes.c_int32 * 3)(0, 0, 0)
+    ref = ogoal.bake(occ.cpu().numpy(), 16.0, np.zeros(3, np.int32), np.zeros(3, np.int32))
+    ws = torch.empty(int(lib.sdfr_goal_workspace_bytes(13, 11, 9)), dtype=torch.uint8, device=dev)
+    q = torch.zeros(n + 8, dtype=torch.int16, device=dev)
+    g = torch.zeros(n + 8, dtype=torch.float32, device=dev)
+    info = _sdfr.GoalInfo()
+    print(f"case goal alignment {shift}", flush=True)
+    rc = lib.sdfr_goal_bake(occ.data_ptr(), 13, 11, 9, 16.0, lo, lo, 1 << 20, q[shift:].data_ptr(),
+                            g[shift:].data_ptr(), ctypes.byref(info), ws.data_ptr(), ws.numel(),
+                            torch.cuda.current_stream().cuda_stream)
+    assert rc == 0
+    assert np.array_equal(q[shift:shift + n].cpu().numpy().view(np.uint16).reshape(shape), ref["grid_q"])
+    assert np.array_equal(g[shift:shift + n].cpu().numpy().reshape(shape), ref["grid"])
+    assert not q[shift + n:].any() and not g[shift + n:].any() and not q[:shift].any()
