@@ -34,7 +34,7 @@ extern "C" {
 
 /* Bumped on every struct or semantic change; the binding refuses a library
  * reporting another value. */
-#define SDFR_ABI_VERSION 13
+#define SDFR_ABI_VERSION 14
 
 /* Element types of caller arrays. */
 enum {
@@ -343,6 +343,15 @@ SDFR_API int32_t sdfr_goal_sample(const void* grid, int32_t grid_dtype, float qu
                                   int32_t ny, int32_t nz, const double* mins, double cell,
                                   double reach_max, const void* pos, int32_t pos_dtype,
                                   int64_t pos_stride, int64_t n, float* out, void* stream);
+
+/* sdfr_goal_yaw: yaw in degrees [0, 360] of the steepest horizontal descent at
+ * n positions, from sdfr_goal_sample's values one cell off along x and y —
+ * GoalField.descent_yaw (goalfield.py:101-107). Arguments and errors as
+ * sdfr_goal_sample's. */
+SDFR_API int32_t sdfr_goal_yaw(const void* grid, int32_t grid_dtype, float quant, int32_t nx,
+                               int32_t ny, int32_t nz, const double* mins, double cell,
+                               double reach_max, const void* pos, int32_t pos_dtype,
+                               int64_t pos_stride, int64_t n, float* out, void* stream);
 SDFR_API const char* sdfr_goal_last_error(void);
 
 /* Message of the calling thread's most recent error ("" if none). */

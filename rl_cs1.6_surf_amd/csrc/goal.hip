@@ -419,21 +419,20 @@ __global__ __launch_bounds__(256) void goal_quantise(const float* d, int64_t vox
 }
 
 // GoalField.sample (goalfield.py:68-94): trilinear over the honest corners.
-template <int GRID, int POS>
-__global__ __launch_bounds__(256) void goal_sample(const void* __restrict__ grid, float quant, int nx,
-                                                   int ny, int nz, double mnx, double mny, double mnz,
-                                                   double cell, float valid_max, float sentinel,
-                                                   const void* __restrict__ pos, int64_t pos_stride,
-                                                   int64_t n, float* __restrict__ out) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    double p[3];
-    for (int j = 0; j < 3; ++j)
-        p[j] = POS == SDFR_F64 ? ((const double*)pos)[i * pos_stride + j]
-                               : (double)((const float*)pos)[i * pos_stride + j];
-    const double gx = (p[0] - mnx) / cell - 0.5;
-    const double gy = (p[1] - mny) / cell - 0.5;
-    const double gz = (p[2] - mnz) / cell - 0.5;
+struct FieldArgs {
+    const void* grid;
+    float quant;
+    int nx, ny, nz;
+    double mnx, mny, mnz, cell;
+    float valid_max, sentinel;
+};
+
+template <int GRID>
+__device__ __forceinline__ float field_at(const FieldArgs& a, double px, double py, double pz) {
+    const int nx = a.nx, ny = a.ny, nz = a.nz;
+    const double gx = (px - a.mnx) / a.cell - 0.5;
+    const double gy = (py - a.mny) / a.cell - 0.5;
+    const double gz = (pz - a.mnz) / a.cell - 0.5;
     const double fx0 = floor(gx), fy0 = floor(gy), fz0 = floor(gz);
     const float fx = (float)(gx - fx0), fy = (float)(gy - fy0), fz = (float)(gz - fz0);
     // corner indices clamped in double: a far-off position cannot overflow
@@ -448,16 +447,57 @@ __global__ __launch_bounds__(256) void goal_sample(const void* __restrict__ grid
 #pragma unroll
             for (int dx = 0; dx < 2; ++dx) {
                 const int64_t k = ((int64_t)cz[dz] * ny + (int64_t)cy[dy]) * nx + (int64_t)cx[dx];
-                const float v = GRID == SDFR_F32 ? ((const float*)grid)[k]
-                                                 : (float)((const uint16_t*)grid)[k] * quant;
+                const float v = GRID == SDFR_F32 ? ((const float*)a.grid)[k]
+                                                 : (float)((const uint16_t*)a.grid)[k] * a.quant;
                 const float wx = dx ? fx : 1.0f - fx;
                 const float wy = dy ? fy : 1.0f - fy;
                 const float wz = dz ? fz : 1.0f - fz;
-                const float w = ((wx * wy) * wz) * (v < valid_max ? 1.0f : 0.0f);
+                const float w = ((wx * wy) * wz) * (v < a.valid_max ? 1.0f : 0.0f);
                 num = num + w * v;
                 den = den + w;
             }
-    out[i] = den > 1e-6f ? num / fmaxf(den, 1e-6f) : sentinel;
+    return den > 1e-6f ? num / fmaxf(den, 1e-6f) : a.sentinel;
+}
+
+template <int POS>
+__device__ __forceinline__ double pos_at(const void* pos, int64_t i) {
+    return POS == SDFR_F64 ? ((const double*)pos)[i] : (double)((const float*)pos)[i];
+}
+
+template <int GRID, int POS>
+__global__ __launch_bounds__(256) void goal_sample(FieldArgs a, const void* __restrict__ pos, int64_t pos_stride,
+                                                   int64_t n, float* __restrict__ out) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const int64_t o = i * pos_stride;
+    out[i] = field_at<GRID>(a, pos_at<POS>(pos, o), pos_at<POS>(pos, o + 1), pos_at<POS>(pos, o + 2));
+}
+
+// GoalField.descent_yaw (goalfield.py:101-107): the yaw of the steepest
+// horizontal descent from samples one cell off along +x, -x, +y and -y. What
+// bounds it at a reservoir's ~1500 positions is launches and round trips to
+// memory, so one launch does what took fifteen (positions to float64, four
+// offset copies, samples, differences, atan2, degrees, remainder): four lanes
+// a position, one sample each, handed over by shuffles, so a position's 32
+// gathers are in flight together. 1500 host positions: 108 us a call before,
+// 47 now, most of it the copies there and back.
+template <int GRID, int POS>
+__global__ __launch_bounds__(256) void goal_yaw(FieldArgs a, const void* __restrict__ pos, int64_t pos_stride,
+                                                int64_t n, float* __restrict__ out) {
+    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x, i = t >> 2;
+    const int dir = (int)(t & 3);
+    // lanes past the end sample the last position: the shuffles want every lane
+    const int64_t o = (i < n ? i : n - 1) * pos_stride;
+    const double h = dir & 1 ? -a.cell : a.cell;
+    const double px = pos_at<POS>(pos, o) + (dir < 2 ? h : 0.0);
+    const double py = pos_at<POS>(pos, o + 1) + (dir < 2 ? 0.0 : h);
+    const float s = field_at<GRID>(a, px, py, pos_at<POS>(pos, o + 2));
+    const float diff = s - __shfl_down(s, 1);   // lane 0 of 4: along x, lane 2: along y
+    const float dx = diff, dy = __shfl_down(diff, 2);
+    if (dir != 0 || i >= n) return;
+    float yaw = fmodf(atan2f(-dy, -dx) * 57.29577951308232f, 360.0f);   // degrees, Python's remainder
+    if (yaw < 0.0f) yaw += 360.0f;
+    out[i] = yaw;
 }
 
 struct Layout {
@@ -610,38 +650,65 @@ SDFR_API int32_t sdfr_goal_bake(const uint8_t* occ, int32_t nx, int32_t ny, int3
     return 0;
 }
 
+// The checks that goal_sample and goal_yaw share; fills `a`.
+static int32_t field_args(const char* fn, FieldArgs* a, const void* grid, int32_t grid_dtype, float quant, int32_t nx,
+                          int32_t ny, int32_t nz, const double* mins, double cell, double reach_max, const void* pos,
+                          int32_t pos_dtype, int64_t pos_stride, int64_t n, const float* out, int per_block) {
+    g_goal_err[0] = '\0';
+    if (!grid || !mins || !out || (!pos && n > 0)) return gfail(-1, "%s: null pointer argument", fn);
+    if (nx <= 0 || ny <= 0 || nz <= 0 || n < 0 || !(cell > 0.0)) return gfail(-2, "%s: bad dims, count or cell", fn);
+    if (grid_dtype != SDFR_F32 && grid_dtype != SDFR_U16)
+        return gfail(-3, "%s: grid dtype must be f32 or u16 (got %d)", fn, grid_dtype);
+    if (pos_dtype != SDFR_F32 && pos_dtype != SDFR_F64)
+        return gfail(-3, "%s: position dtype must be f32 or f64 (got %d)", fn, pos_dtype);
+    if (pos_stride < 3) return gfail(-2, "%s: position row stride below 3", fn);
+    if (n > (int64_t)0x7fffffff * per_block) return gfail(-2, "%s: too many positions", fn);
+    // GoalField.__init__ (goalfield.py:59-66): Python floats, compared in fp32
+    *a = {grid, quant, nx, ny, nz, mins[0], mins[1], mins[2], cell,
+          (float)(reach_max + 0.5 * cell), (float)(reach_max + 2.0 * cell)};
+    return 0;
+}
+
+#define GOAL_LAUNCH(KERNEL, PER_BLOCK)                                                             \
+    do {                                                                                           \
+        const int blocks = (int)((n + (PER_BLOCK)-1) / (PER_BLOCK));                               \
+        hipStream_t st = (hipStream_t)stream;                                                      \
+        if (grid_dtype == SDFR_F32 && pos_dtype == SDFR_F64)                                       \
+            KERNEL<SDFR_F32, SDFR_F64><<<blocks, 256, 0, st>>>(a, pos, pos_stride, n, out);        \
+        else if (grid_dtype == SDFR_F32)                                                           \
+            KERNEL<SDFR_F32, SDFR_F32><<<blocks, 256, 0, st>>>(a, pos, pos_stride, n, out);        \
+        else if (pos_dtype == SDFR_F64)                                                            \
+            KERNEL<SDFR_U16, SDFR_F64><<<blocks, 256, 0, st>>>(a, pos, pos_stride, n, out);        \
+        else                                                                                       \
+            KERNEL<SDFR_U16, SDFR_F32><<<blocks, 256, 0, st>>>(a, pos, pos_stride, n, out);        \
+    } while (0)
+
 SDFR_API int32_t sdfr_goal_sample(const void* grid, int32_t grid_dtype, float quant, int32_t nx,
                                   int32_t ny, int32_t nz, const double* mins, double cell,
                                   double reach_max, const void* pos, int32_t pos_dtype,
                                   int64_t pos_stride, int64_t n, float* out, void* stream) {
-    g_goal_err[0] = '\0';
-    if (!grid || !mins || !out || (!pos && n > 0))
-        return gfail(-1, "sdfr_goal_sample: null pointer argument");
-    if (nx <= 0 || ny <= 0 || nz <= 0 || n < 0 || !(cell > 0.0))
-        return gfail(-2, "sdfr_goal_sample: bad dims, count or cell");
-    if (grid_dtype != SDFR_F32 && grid_dtype != SDFR_U16)
-        return gfail(-3, "sdfr_goal_sample: grid dtype must be f32 or u16 (got %d)", grid_dtype);
-    if (pos_dtype != SDFR_F32 && pos_dtype != SDFR_F64)
-        return gfail(-3, "sdfr_goal_sample: position dtype must be f32 or f64 (got %d)", pos_dtype);
-    if (pos_stride < 3) return gfail(-2, "sdfr_goal_sample: position row stride below 3");
-    if (n == 0) return 0;
-    if (n > (int64_t)0x7fffffff * 256) return gfail(-2, "sdfr_goal_sample: too many positions");
-    // GoalField.__init__ (goalfield.py:59-66): Python floats, compared in fp32
-    const float sentinel = (float)(reach_max + 2.0 * cell);
-    const float valid_max = (float)(reach_max + 0.5 * cell);
-    const int blocks = (int)((n + 255) / 256);
-    hipStream_t st = (hipStream_t)stream;
-#define GOAL_SAMPLE(G, P)                                                                              \
-    goal_sample<G, P><<<blocks, 256, 0, st>>>(grid, quant, nx, ny, nz, mins[0], mins[1], mins[2], cell, \
-                                              valid_max, sentinel, pos, pos_stride, n, out)
-    if (grid_dtype == SDFR_F32 && pos_dtype == SDFR_F64) GOAL_SAMPLE(SDFR_F32, SDFR_F64);
-    else if (grid_dtype == SDFR_F32) GOAL_SAMPLE(SDFR_F32, SDFR_F32);
-    else if (pos_dtype == SDFR_F64) GOAL_SAMPLE(SDFR_U16, SDFR_F64);
-    else GOAL_SAMPLE(SDFR_U16, SDFR_F32);
-#undef GOAL_SAMPLE
+    FieldArgs a;
+    const int32_t rc = field_args("sdfr_goal_sample", &a, grid, grid_dtype, quant, nx, ny, nz, mins, cell, reach_max,
+                                  pos, pos_dtype, pos_stride, n, out, 256);
+    if (rc != 0 || n == 0) return rc;
+    GOAL_LAUNCH(goal_sample, 256);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return gfail(-4, "sdfr_goal_sample: launch failed: %s", hipGetErrorString(e));
     return 0;
 }
+
+SDFR_API int32_t sdfr_goal_yaw(const void* grid, int32_t grid_dtype, float quant, int32_t nx, int32_t ny, int32_t nz,
+                               const double* mins, double cell, double reach_max, const void* pos, int32_t pos_dtype,
+                               int64_t pos_stride, int64_t n, float* out, void* stream) {
+    FieldArgs a;
+    const int32_t rc = field_args("sdfr_goal_yaw", &a, grid, grid_dtype, quant, nx, ny, nz, mins, cell, reach_max, pos,
+                                  pos_dtype, pos_stride, n, out, 64);
+    if (rc != 0 || n == 0) return rc;
+    GOAL_LAUNCH(goal_yaw, 64);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return gfail(-4, "sdfr_goal_yaw: launch failed: %s", hipGetErrorString(e));
+    return 0;
+}
+#undef GOAL_LAUNCH
 
 }  // extern "C"

@@ -18,7 +18,7 @@ import torch  # noqa: F401  (load torch's HIP runtime first, see above)
 PKG_ROOT = Path(__file__).resolve().parents[1]
 LIB_PATH = PKG_ROOT / "lib" / "libsdfr.so"
 
-ABI_VERSION = 13
+ABI_VERSION = 14
 NOALLOC_SCRATCH_BYTES = 24 << 20   # SDFR_NOALLOC_SCRATCH_BYTES
 
 # element types (SDFR_* in sdfr.h)
@@ -37,7 +37,7 @@ EXPORTS = ("sdfr_abi_version", "sdfr_last_error", "sdfr_grid_create", "sdfr_grid
            "sdfr_grid_read",
            "sdfr_edt_workspace_bytes",
            "sdfr_edt", "sdfr_edt_last_error", "sdfr_goal_workspace_bytes", "sdfr_goal_bake",
-           "sdfr_goal_sample", "sdfr_goal_last_error")
+           "sdfr_goal_sample", "sdfr_goal_yaw", "sdfr_goal_last_error")
 
 
 class GridDesc(ctypes.Structure):
@@ -143,6 +143,8 @@ def load(path: Path | str | None = None):
     lib.sdfr_goal_sample.argtypes = [vp, i32, ctypes.c_float, i32, i32, i32,
                                      ctypes.POINTER(ctypes.c_double), ctypes.c_double,
                                      ctypes.c_double, vp, i32, i64, i64, vp, vp]
+    lib.sdfr_goal_yaw.restype = i32
+    lib.sdfr_goal_yaw.argtypes = lib.sdfr_goal_sample.argtypes
     lib.sdfr_goal_last_error.restype = ctypes.c_char_p
     lib.sdfr_goal_last_error.argtypes = []
     got = lib.sdfr_abi_version()

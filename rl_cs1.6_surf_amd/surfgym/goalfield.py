@@ -140,7 +140,9 @@ class GoalField:
         p = torch.from_numpy(np.ascontiguousarray(a.reshape(-1, 3))).to(self.device)
         return p, _sdfr.F64, 3, True
 
-    def _sample_dev(self, p, code, stride) -> torch.Tensor:
+    def _at(self, entry: str, p, code, stride) -> torch.Tensor:
+        """One launch of the field's C entry ``entry`` over positions from
+        :meth:`_positions`: (n,) float32 on the device."""
         lib = _sdfr.load()
         n = int(p.shape[0])
         out = torch.empty(n, dtype=torch.float32, device=self.device)
@@ -148,12 +150,12 @@ class GoalField:
             return out
         with torch.cuda.device(self.device):
             stream = torch.cuda.current_stream(self.device).cuda_stream
-            rc = lib.sdfr_goal_sample(self._grid.data_ptr(), self._kind, float(self.quant),
-                                      int(self.dims[0]), int(self.dims[1]), int(self.dims[2]),
-                                      self._mins_c, self.cell, self.reach_max,
-                                      p.data_ptr(), code, int(stride), n, out.data_ptr(), stream)
+            rc = getattr(lib, entry)(self._grid.data_ptr(), self._kind, float(self.quant),
+                                     int(self.dims[0]), int(self.dims[1]), int(self.dims[2]),
+                                     self._mins_c, self.cell, self.reach_max,
+                                     p.data_ptr(), code, int(stride), n, out.data_ptr(), stream)
         if rc != 0:
-            raise _sdfr.SdfrError(f"sdfr_goal_sample failed ({rc}): "
+            raise _sdfr.SdfrError(f"{entry} failed ({rc}): "
                                   f"{lib.sdfr_goal_last_error().decode('utf-8', 'replace')}")
         return out
 
@@ -163,7 +165,7 @@ class GoalField:
         (goalfield.py:68-94). numpy in, numpy out; a device tensor in, a
         device tensor out (no host synchronisation)."""
         p, code, stride, was_np = self._positions(pos)
-        out = self._sample_dev(p, code, stride)
+        out = self._at("sdfr_goal_sample", p, code, stride)
         return out.cpu().numpy() if was_np else out
 
     def reachable(self, pos):
@@ -174,17 +176,13 @@ class GoalField:
 
     def descent_yaw(self, pos):
         """Yaw in degrees of the steepest horizontal descent
-        (goalfield.py:101-107): one launch samples p +- cell along x and y."""
-        p, _, _, was_np = self._positions(pos)
-        p = p[:, :3].to(torch.float64)
-        h = self.cell
-        off = torch.tensor([[h, 0, 0], [-h, 0, 0], [0, h, 0], [0, -h, 0]], dtype=torch.float64,
-                           device=self.device)
-        q = (p[None, :, :] + off[:, None, :]).reshape(-1, 3).contiguous()
-        s = self._sample_dev(q, _sdfr.F64, 3).view(4, -1)
-        dx = s[0] - s[1]
-        dy = s[2] - s[3]
-        yaw = torch.remainder(torch.rad2deg(torch.atan2(-dy, -dx)), 360.0)
+        (goalfield.py:101-107): one launch samples p +- cell along x and y
+        and turns the differences into degrees."""
+        p, code, stride, was_np = self._positions(pos)
+        if p.shape[0] == 0:
+            raise RuntimeError("descent_yaw needs at least one position")
+        # (only a single row, whose stride is not used, can have one below 3)
+        yaw = self._at("sdfr_goal_yaw", p, code, max(stride, 3))
         return yaw.cpu().numpy() if was_np else yaw
 
 
