@@ -55,6 +55,7 @@ __attribute__((format(printf, 2, 3))) int32_t gfail(int32_t code, const char* fm
 }
 
 constexpr int kT = 8;                    // tile edge (voxels)
+constexpr int kTileVox = kT * kT * kT;
 constexpr int kH = kT + 2;               // tile edge with halo
 // LDS floats per column (8 and a gap) and per row of columns: 16-byte reads of
 // 8 lanes along x fall 12 words apart, and 32 mod 64 from the next row's, so
@@ -75,7 +76,8 @@ enum { kCount0 = 0, kCount1 = 1, kCount2 = 2, kSeeds = 3, kReach = 4, kLastBusy 
 
 struct GoalArgs {
     const uint8_t* occ;
-    float* d;
+    float* d;             // [tiles][y][x][z], kTileVox a tile; +inf past the grid's edge
+    uint64_t* open;       // [tiles][kT]: plane z's free voxels inside the grid, bit 8 * y + x
     uint32_t* mark;       // [tiles] last sweep the tile was queued for
     uint32_t* queues;     // [2][parts][part_cap], sweep k reads [k & 1]
     uint32_t* counts;     // [3][parts], part_pitch words apart: sweep k's is [k % 3]
@@ -88,9 +90,9 @@ struct GoalArgs {
     float w1, w2, w3;     // edge weights for |o|^2 = 1, 2, 3
 };
 
-// Which of 8 queues a tile goes to. A tile's rows (and halo) use 40 of each
-// 128-byte line they touch, so tiles that share lines are kept in one queue,
-// whose sweep blocks run on one XCD (block b on XCD b % 8) and share its L2:
+// Which of 8 queues a tile goes to. A tile's halo lies in its neighbours'
+// lines, so near tiles are kept in one queue, whose sweep blocks run on one
+// XCD (block b on XCD b % 8) and share its L2:
 // blocks of 4 x 2 x 2 tiles, dealt out in order over rows made odd in length,
 // so that neighbours along every axis go to different queues.
 __device__ __forceinline__ uint32_t part_of(const GoalArgs& a, int tx, int ty, int tz) {
@@ -108,52 +110,49 @@ __device__ __forceinline__ uint32_t* queue_of(const GoalArgs& a, uint32_t k, uin
 }
 
 // d = +inf everywhere, 0 on the free voxels of the seed box; the tiles that
-// hold a seed or touch one through their halo form the first queue. Four
-// distances per store (the distances start the workspace, which the bake
-// requires 64-byte aligned).
+// hold a seed or touch one through their halo form the first queue. Tiles
+// without a free voxel are marked as if queued for good: no visit could lower
+// anything there. A wave a tile, a lane a column.
 __global__ __launch_bounds__(256) void goal_init(GoalArgs a, int lx, int ly, int lz, int hx, int hy,
                                                  int hz, int tlx, int tly, int tlz, int thx, int thy,
                                                  int thz) {
-    const int64_t vox = (int64_t)a.nx * a.ny * a.nz, n4 = (vox + 3) >> 2;
-    const int64_t step = (int64_t)gridDim.x * blockDim.x, first = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int lane = threadIdx.x & 63;
     uint32_t seeds = 0;
-    auto value = [&](int64_t i, int x, int y, int z) {
-        const bool seed = x >= lx && x <= hx && y >= ly && y <= hy && z >= lz && z <= hz && !a.occ[i];
-        seeds += seed;
-        return seed ? 0.0f : INFINITY;
-    };
-    for (int64_t i = first; i < n4; i += step) {
-        const int64_t v0 = i << 2, r = v0 / a.nx;
-        int x = (int)(v0 - r * a.nx), y = (int)(r % a.ny), z = (int)(r / a.ny);
-        float v[4];
+    for (uint32_t t = blockIdx.x * 4 + (threadIdx.x >> 6); t < a.tiles; t += gridDim.x * 4) {
+        const int tx = (int)(t % (uint32_t)a.tx);
+        const uint32_t r = t / (uint32_t)a.tx;
+        const int ty = (int)(r % (uint32_t)a.ty), tz = (int)(r / (uint32_t)a.ty);
+        const int x = tx * kT + (lane & 7), y = ty * kT + (lane >> 3), z0 = tz * kT;
+        const bool inside = x < a.nx && y < a.ny;
+        const bool box = x >= lx && x <= hx && y >= ly && y <= hy;
+        const int64_t idx = ((int64_t)z0 * a.ny + y) * a.nx + x, plane = (int64_t)a.ny * a.nx;
+        float v[kT];
+        uint64_t mine = 0, some = 0;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            v[j] = v0 + j < vox ? value(v0 + j, x, y, z) : 0.0f;
-            if (++x == a.nx) {
-                x = 0;
-                if (++y == a.ny) {
-                    y = 0;
-                    ++z;
-                }
-            }
+        for (int z = 0; z < kT; ++z) {
+            const bool free = inside && z0 + z < a.nz && a.occ[idx + z * plane] == 0;
+            const bool seed = free && box && z0 + z >= lz && z0 + z <= hz;
+            const uint64_t m = __ballot(free);
+            if (lane == z) mine = m;
+            some |= m;
+            seeds += seed;
+            v[z] = seed ? 0.0f : INFINITY;
         }
-        if (v0 + 3 < vox) *(float4*)(a.d + v0) = make_float4(v[0], v[1], v[2], v[3]);
-        else
-            for (int j = 0; v0 + j < vox; ++j) a.d[v0 + j] = v[j];
-    }
-    for (int64_t t = first; t < a.tiles; t += step) {
-        const int tx = (int)(t % a.tx);
-        const int64_t r = t / a.tx;
-        const int ty = (int)(r % a.ty), tz = (int)(r / a.ty);
-        const bool in = tx >= tlx && tx <= thx && ty >= tly && ty <= thy && tz >= tlz && tz <= thz;
-        a.mark[t] = in ? 1u : 0u;
-        if (in) {
-            const uint32_t part = part_of(a, tx, ty, tz);
-            queue_of(a, 1u, part)[atomicAdd(count_of(a, 1u, part), 1u)] = (uint32_t)t;
+        float4* col = (float4*)(a.d + (int64_t)t * kTileVox + lane * kT);
+        col[0] = make_float4(v[0], v[1], v[2], v[3]);
+        col[1] = make_float4(v[4], v[5], v[6], v[7]);
+        if (lane < kT) a.open[(int64_t)t * kT + lane] = mine;
+        if (lane == 0) {
+            const bool in = tx >= tlx && tx <= thx && ty >= tly && ty <= thy && tz >= tlz && tz <= thz;
+            a.mark[t] = some == 0 ? ~0u : in ? 1u : 0u;
+            if (in && some) {
+                const uint32_t part = part_of(a, tx, ty, tz);
+                queue_of(a, 1u, part)[atomicAdd(count_of(a, 1u, part), 1u)] = t;
+            }
         }
     }
     for (int off = 32; off > 0; off >>= 1) seeds += __shfl_down(seeds, off);
-    if ((threadIdx.x & 63) == 0 && seeds) atomicAdd(&a.ctl[kSeeds], seeds);
+    if (lane == 0 && seeds) atomicAdd(&a.ctl[kSeeds], seeds);
 }
 
 // The smaller of two distances: of non-negative floats (+inf among them) as
@@ -191,18 +190,23 @@ __device__ __forceinline__ void wave_sync() {
 // instructions a voxel instead of 26 and 52). Up and down its own column a
 // lane relaxes in order, so a value crosses the tile along z in one pass.
 //
-// What bounds it: in the ~20 long sweeps of a bake the lines the tiles read
-// (240 misses a visit with tiles dealt to any XCD, 3.6 TB/s; queues by XCD
-// took the longest from 39 to 27 us), in the ~40 short ones the chain of
-// round trips to memory of one visit (queue, tile, mark, slot: 8-11 us).
-// 256x256x128 voxels, 58 sweeps: 29 us a sweep with a block of 512 threads
-// and 26 LDS reads a voxel, 18 with a wave a tile, 16 with the columns loaded
-// straight to their lanes, 13 with a queue per XCD. Also measured: flags per
-// tile instead of queues (no claims, but a static deal of tiles to waves: 28
-// us), reading a mark before its atomic (+2 us), no order along z (+2 us),
-// queueing only tiles whose halo copy would fall (20% fewer visits, each 3 us
-// longer).
-__global__ __launch_bounds__(kThreads) void goal_sweep(GoalArgs a, uint32_t k) {
+// The distances lie tile by tile, each column's 8 voxels together, so a lane
+// takes a column in two 16-byte loads (8 loads a visit with the halo, ~100
+// lines; rows of the grid took 28 loads and 240 lines), and the free voxels
+// are lane masks in scalar registers.
+//
+// What bounds it: in the ~20 long sweeps of a bake (up to 5000 visits, one a
+// wave) vector issue and LDS reads of the ~10 relaxations of a visit, in the
+// ~30 short ones the chain of round trips to memory of one visit (queue, tile,
+// mark, slot: ~6 us). 256x256x128 voxels, 50 sweeps: 29 us a sweep with a block
+// of 512 threads and 26 LDS reads a voxel, 18 with a wave a tile, 16 with the
+// columns loaded straight to their lanes; a whole bake 1086 us with a queue
+// per XCD, 887 with the distances by tile. Also measured: flags per tile
+// instead of queues (no claims, but a static deal of tiles to waves: 28 us),
+// reading a mark before its atomic (+2 us), no order along z (+2 us), queueing
+// only tiles whose halo copy would fall (20% fewer visits, each 3 us longer).
+__global__ __launch_bounds__(kThreads) void goal_sweep(GoalArgs a, const uint64_t* __restrict__ open_planes,
+                                                       uint32_t k) {
     __shared__ __align__(16) float s_all[kWaves][kTileLds];
     const uint32_t part = blockIdx.x % (uint32_t)a.parts, block = blockIdx.x / (uint32_t)a.parts;
     const uint32_t blocks = gridDim.x / (uint32_t)a.parts;   // of this queue
@@ -234,42 +238,49 @@ __global__ __launch_bounds__(kThreads) void goal_sweep(GoalArgs a, uint32_t k) {
     const int rx = side == 0 ? 0 : side == 1 ? kH - 1 : side > 3 ? (lane & 1) * (kH - 1) : at;
     const int ry = side == 2 ? 0 : side == 3 ? kH - 1 : side > 3 ? ((lane >> 1) & 1) * (kH - 1) : at;
     float* ring = s + ry * kRow + rx * kCol;
+    // ... from the tile its column lies in
+    const int rtx = rx == 0 ? -1 : rx == kH - 1 ? 1 : 0, rty = ry == 0 ? -1 : ry == kH - 1 ? 1 : 0;
+    const int rcol = ((ry - 1) & 7) * kT + ((rx - 1) & 7);
+    const int64_t layer = (int64_t)a.tx * a.ty * kTileVox;   // distances to the tile above
+    const int64_t roff = ((int64_t)rty * a.tx + rtx) * kTileVox + rcol * kT;
     for (; e < n; e += blocks * kWaves, tile_v = e < n ? qi[e] : 0u) {
         const uint32_t tile = __builtin_amdgcn_readfirstlane(tile_v);
         const int tx = (int)(tile % (uint32_t)a.tx);
         const uint32_t r = tile / (uint32_t)a.tx;
         const int ty = (int)(r % (uint32_t)a.ty), tz = (int)(r / (uint32_t)a.ty);
-        const int x0 = tx * kT, y0 = ty * kT, z0 = tz * kT;
-        const int x = x0 + lx, y = y0 + ly, xr = x0 + rx - 1, yr = y0 + ry - 1;
-        const bool inside = x < a.nx && y < a.ny;
-        const bool on_ring = lane < 36 && xr >= 0 && yr >= 0 && xr < a.nx && yr < a.ny;
-        const int64_t idx = ((int64_t)z0 * a.ny + y) * a.nx + x, plane = (int64_t)a.ny * a.nx;
-        const int64_t rdx = ((int64_t)z0 * a.ny + yr) * a.nx + xr;
+        const bool on_ring = lane < 36 && tx + rtx >= 0 && tx + rtx < a.tx && ty + rty >= 0 && ty + rty < a.ty;
         // the lane's own column and its halo column, both with the voxels
         // below and above; outside the grid nothing lowers a neighbour
-        float cv[kH], rv[kH];
-        bool open[kT];
-#pragma unroll
-        for (int z = 0; z < kH; ++z) {
-            const bool in_z = z0 + z - 1 >= 0 && z0 + z - 1 < a.nz;   // uniform
-            cv[z] = rv[z] = INFINITY;
-            if (in_z && inside) cv[z] = a.d[idx + (z - 1) * plane];
-            if (in_z && on_ring) rv[z] = a.d[rdx + (z - 1) * plane];
+        float* home = a.d + (int64_t)tile * kTileVox + lane * kT;
+        const float* rim = a.d + (int64_t)tile * kTileVox + roff;
+        const float4 inf4 = make_float4(INFINITY, INFINITY, INFINITY, INFINITY);
+        const float4 c0 = ((const float4*)home)[0], c1 = ((const float4*)home)[1];
+        const float4 r0 = on_ring ? ((const float4*)rim)[0] : inf4, r1 = on_ring ? ((const float4*)rim)[1] : inf4;
+        float cb = INFINITY, ca = INFINITY, rb = INFINITY, ra = INFINITY;
+        if (tz > 0) {   // uniform
+            cb = home[kT - 1 - layer];
+            if (on_ring) rb = rim[kT - 1 - layer];
         }
+        if (tz + 1 < a.tz) {
+            ca = home[layer];
+            if (on_ring) ra = rim[layer];
+        }
+        const float cv[kT] = {c0.x, c0.y, c0.z, c0.w, c1.x, c1.y, c1.z, c1.w};
+        uint64_t open[kT];
 #pragma unroll
-        for (int z = 0; z < kT; ++z) open[z] = inside && z0 + z < a.nz && a.occ[idx + z * plane] == 0;
+        for (int z = 0; z < kT; ++z) open[z] = open_planes[(int64_t)tile * kT + z];
         float start[kT], cur[kT];
 #pragma unroll
-        for (int z = 0; z < kT; ++z) start[z] = cur[z] = cv[z + 1];
-        *(float4*)own = make_float4(cv[1], cv[2], cv[3], cv[4]);
-        *(float4*)(own + 4) = make_float4(cv[5], cv[6], cv[7], cv[8]);
-        zlo[c] = cv[0];
-        zhi[c] = cv[kH - 1];
+        for (int z = 0; z < kT; ++z) start[z] = cur[z] = cv[z];
+        *(float4*)own = c0;
+        *(float4*)(own + 4) = c1;
+        zlo[c] = cb;
+        zhi[c] = ca;
         if (lane < 36) {
-            *(float4*)ring = make_float4(rv[1], rv[2], rv[3], rv[4]);
-            *(float4*)(ring + 4) = make_float4(rv[5], rv[6], rv[7], rv[8]);
-            zlo[ry * kH + rx] = rv[0];
-            zhi[ry * kH + rx] = rv[kH - 1];
+            *(float4*)ring = r0;
+            *(float4*)(ring + 4) = r1;
+            zlo[ry * kH + rx] = rb;
+            zhi[ry * kH + rx] = ra;
         }
         wave_sync();
         // what the planes below and above give the first and last voxel
@@ -308,10 +319,10 @@ __global__ __launch_bounds__(kThreads) void goal_sweep(GoalArgs a, uint32_t k) {
                 m[z] = least(least(cur[z], least(f[z] + w1, g[z] + w2)),
                              least(z ? q[z - 1] : below, z < kT - 1 ? q[z + 1] : above));
                 if (z) m[z] = least(m[z], m[z - 1] + w1);
-                m[z] = open[z] ? m[z] : INFINITY;
+                m[z] = __builtin_amdgcn_inverse_ballot_w64(open[z]) ? m[z] : INFINITY;
             }
 #pragma unroll
-            for (int z = kT - 2; z >= 0; --z) m[z] = open[z] ? least(m[z], m[z + 1] + w1) : INFINITY;
+            for (int z = kT - 2; z >= 0; --z) m[z] = __builtin_amdgcn_inverse_ballot_w64(open[z]) ? least(m[z], m[z + 1] + w1) : INFINITY;
             bool lowered = false;
 #pragma unroll
             for (int z = 0; z < kT; ++z) {
@@ -327,11 +338,10 @@ __global__ __launch_bounds__(kThreads) void goal_sweep(GoalArgs a, uint32_t k) {
         }
         bool any = false;
 #pragma unroll
-        for (int z = 0; z < kT; ++z) {
-            if (cur[z] < start[z]) {
-                a.d[idx + z * plane] = cur[z];
-                any = true;
-            }
+        for (int z = 0; z < kT; ++z) any |= cur[z] < start[z];
+        if (any) {   // no other wave writes this tile in this sweep
+            ((float4*)home)[0] = make_float4(cur[0], cur[1], cur[2], cur[3]);
+            ((float4*)home)[1] = make_float4(cur[4], cur[5], cur[6], cur[7]);
         }
         // neighbour tiles whose halo holds a lowered voxel; lane t < 27 looks
         // after direction t
@@ -353,17 +363,15 @@ __global__ __launch_bounds__(kThreads) void goal_sweep(GoalArgs a, uint32_t k) {
 }
 
 // reach_max: the largest finite distance (non-negative floats order as their
-// bit patterns). Four distances per load (the distances start the workspace,
-// which the bake requires 64-byte aligned), the last vox % 4 one at a time;
-// one atomic per block (atomics from every wave to the one word serialise).
+// bit patterns). Four distances per load over whole tiles (+inf past the
+// grid's edge); one atomic per block (atomics from every wave to the one word
+// serialise).
 constexpr int kReachBlocks = 512;
-__global__ __launch_bounds__(256) void goal_reach_max(GoalArgs a, int64_t vox) {
-    const float* d = a.d;
+__global__ __launch_bounds__(256) void goal_reach_max(GoalArgs a) {
     __shared__ uint32_t s_m[4];
-
     uint32_t m = 0;
-    const int64_t n4 = vox >> 2;
-    const float4* d4 = reinterpret_cast<const float4*>(d);
+    const int64_t n4 = (int64_t)a.tiles * (kTileVox / 4);
+    const float4* d4 = reinterpret_cast<const float4*>(a.d);
     const int64_t step = (int64_t)gridDim.x * blockDim.x;
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n4; i += step) {
         const float4 v = d4[i];
@@ -371,10 +379,6 @@ __global__ __launch_bounds__(256) void goal_reach_max(GoalArgs a, int64_t vox) {
         if (v.y != INFINITY) m = max(m, __float_as_uint(v.y));
         if (v.z != INFINITY) m = max(m, __float_as_uint(v.z));
         if (v.w != INFINITY) m = max(m, __float_as_uint(v.w));
-    }
-    for (int64_t i = (n4 << 2) + (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < vox; i += step) {
-        const float v = d[i];
-        if (v != INFINITY) m = max(m, __float_as_uint(v));
     }
     for (int off = 32; off > 0; off >>= 1) m = max(m, (uint32_t)__shfl_down(m, off));
     if ((threadIdx.x & 63) == 0) s_m[threadIdx.x >> 6] = m;
@@ -390,31 +394,59 @@ __global__ __launch_bounds__(256) void goal_reach_max(GoalArgs a, int64_t vox) {
 // d * (1/quant) with the reciprocal rounded to fp32 (identical to d / quant
 // for the power-of-two cells the reference picks), and rounds half to even.
 // The sentinel is the host's reach_max + 2*cell, from the largest distance
-// goal_reach_max left; a field beyond the uint16 range writes nothing. Four
-// voxels a thread (`wide`: the outputs are aligned for it).
-__global__ __launch_bounds__(256) void goal_quantise(const float* d, int64_t vox, const uint32_t* reach, double cell,
-                                                     float inv_quant, float quant, uint16_t* q_out,
-                                                     float* g_out, int wide) {
-    const double sentinel_d = (double)__uint_as_float(*reach) + 2.0 * cell;
+// goal_reach_max left; a field beyond the uint16 range writes nothing. A block
+// turns four tiles along x into rows of 32 voxels through LDS (rows 36 words
+// apart: the 64 columns of a wave then fall on 64 banks), so that both
+// outputs are written in whole lines, four voxels a thread (`wide`: rows and
+// outputs are aligned for it).
+__global__ __launch_bounds__(256) void goal_quantise(GoalArgs a, double cell, float inv_quant, float quant,
+                                                     uint16_t* q_out, float* g_out, int wide) {
+    constexpr int kSpan = 4 * kT, kPitch = kSpan + 4;
+    __shared__ __align__(16) float s[kT * kT * kPitch];
+    const double sentinel_d = (double)__uint_as_float(a.ctl[kReach]) + 2.0 * cell;
     if (sentinel_d / (cell / 8.0) > 65535.0) return;
     const float sentinel = (float)sentinel_d;
     auto code = [&](float v) {
         if (v == INFINITY) v = sentinel;
         return (uint16_t)fminf(fmaxf(rintf(v * inv_quant), 0.0f), 65535.0f);
     };
-    const int64_t step = (int64_t)gridDim.x * blockDim.x, first = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int64_t n4 = wide ? vox >> 2 : 0;
-    for (int64_t i = first; i < n4; i += step) {
-        const float4 v = ((const float4*)d)[i];
-        const ushort4 u = make_ushort4(code(v.x), code(v.y), code(v.z), code(v.w));
-        if (q_out) ((ushort4*)q_out)[i] = u;
-        if (g_out)
-            ((float4*)g_out)[i] = make_float4((float)u.x * quant, (float)u.y * quant, (float)u.z * quant, (float)u.w * quant);
-    }
-    for (int64_t i = (n4 << 2) + first; i < vox; i += step) {
-        const uint16_t u = code(d[i]);
-        if (q_out) q_out[i] = u;
-        if (g_out) g_out[i] = (float)u * quant;
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const uint32_t spans = (uint32_t)(a.tx + 3) / 4u, groups = spans * (uint32_t)a.ty * (uint32_t)a.tz;
+    for (uint32_t gr = blockIdx.x; gr < groups; gr += gridDim.x) {
+        const uint32_t row = gr / spans;   // of tiles: tz * ty_count + ty
+        const int tx0 = (int)(gr - row * spans) * 4;
+        const int ty = (int)(row % (uint32_t)a.ty), tz = (int)(row / (uint32_t)a.ty);
+        if (tx0 + wave < a.tx) {
+            const float4* col = (const float4*)(a.d + ((int64_t)row * a.tx + tx0 + wave) * kTileVox + lane * kT);
+            const float4 lo = col[0], hi = col[1];
+            const float v[kT] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+#pragma unroll
+            for (int z = 0; z < kT; ++z) s[(z * kT + (lane >> 3)) * kPitch + wave * kT + (lane & 7)] = v[z];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const int line = j * 32 + (int)(threadIdx.x >> 3), c = (int)(threadIdx.x & 7) * 4;
+            const int x = tx0 * kT + c, y = ty * kT + (line & 7), z = tz * kT + (line >> 3);
+            if (x >= a.nx || y >= a.ny || z >= a.nz) continue;
+            const int64_t i = ((int64_t)z * a.ny + y) * a.nx + x;
+            const float* v = s + line * kPitch + c;
+            if (wide) {
+                const float4 f = *(const float4*)v;
+                const ushort4 u = make_ushort4(code(f.x), code(f.y), code(f.z), code(f.w));
+                if (q_out) *(ushort4*)(q_out + i) = u;
+                if (g_out)
+                    *(float4*)(g_out + i) =
+                        make_float4((float)u.x * quant, (float)u.y * quant, (float)u.z * quant, (float)u.w * quant);
+            } else {
+                for (int o = 0; o < 4 && x + o < a.nx; ++o) {
+                    const uint16_t u = code(v[o]);
+                    if (q_out) q_out[i + o] = u;
+                    if (g_out) g_out[i + o] = (float)u * quant;
+                }
+            }
+        }
+        __syncthreads();
     }
 }
 
@@ -501,17 +533,17 @@ __global__ __launch_bounds__(256) void goal_yaw(FieldArgs a, const void* __restr
 }
 
 struct Layout {
-    int64_t vox, d_off, mark_off, q_off, ctl_off, total;
+    int64_t d_off, open_off, mark_off, q_off, ctl_off, total;
     uint32_t tiles;
 };
 
 Layout layout_of(int nx, int ny, int nz) {
     Layout l;
-    l.vox = (int64_t)nx * ny * nz;
     const int64_t tiles = (int64_t)((nx + kT - 1) / kT) * ((ny + kT - 1) / kT) * ((nz + kT - 1) / kT);
     l.tiles = (uint32_t)tiles;
     l.d_off = 0;
-    l.mark_off = l.d_off + l.vox * 4;
+    l.open_off = l.d_off + tiles * kTileVox * 4;
+    l.mark_off = l.open_off + tiles * kT * 8;
     l.q_off = l.mark_off + tiles * 4;
     l.ctl_off = l.q_off + 3 * tiles * 4;
     l.ctl_off = (l.ctl_off + 63) & ~(int64_t)63;
@@ -566,6 +598,7 @@ SDFR_API int32_t sdfr_goal_bake(const uint8_t* occ, int32_t nx, int32_t ny, int3
     GoalArgs g;
     g.occ = occ;
     g.d = (float*)(ws + L.d_off);
+    g.open = (uint64_t*)(ws + L.open_off);
     g.mark = (uint32_t*)(ws + L.mark_off);
     g.queues = (uint32_t*)(ws + L.q_off);
     g.ctl = (uint32_t*)(ws + L.ctl_off);
@@ -598,8 +631,8 @@ SDFR_API int32_t sdfr_goal_bake(const uint8_t* occ, int32_t nx, int32_t ny, int3
     uint32_t* const dev_words = g.ctl - (shared - kCtl);
     hipError_t e = hipMemcpyAsync(dev_words, host, shared * 4, hipMemcpyHostToDevice, st);
     if (e != hipSuccess) return gfail(-4, "sdfr_goal_bake: %s", hipGetErrorString(e));
-    const int64_t fours = (L.vox + 1023) / 1024;   // four voxels a thread
-    const int init_blocks = (int)(fours > 8192 ? 8192 : fours);
+    const uint32_t quads = (L.tiles + 3) / 4;   // four tiles a block
+    const int init_blocks = (int)(quads > 8192 ? 8192 : quads);
     goal_init<<<init_blocks, 256, 0, st>>>(g, lo[0], lo[1], lo[2], hi[0], hi[1], hi[2], tlo[0], tlo[1],
                                            tlo[2], thi[0], thi[1], thi[2]);
     int dev = 0, cus = 256;
@@ -611,7 +644,7 @@ SDFR_API int32_t sdfr_goal_bake(const uint8_t* occ, int32_t nx, int32_t ny, int3
     bool done = false;
     while (!done && (int64_t)k <= max_sweeps) {
         for (int j = 0; j < kSweepChunk && (int64_t)k <= max_sweeps; ++j, ++k)
-            goal_sweep<<<sweep_blocks, kThreads, 0, st>>>(g, k);
+            goal_sweep<<<sweep_blocks, kThreads, 0, st>>>(g, g.open, k);
         e = hipGetLastError();
         if (e == hipSuccess) e = hipMemcpyAsync(host, dev_words, shared * 4, hipMemcpyDeviceToHost, st);
         if (e == hipSuccess) e = hipStreamSynchronize(st);
@@ -623,13 +656,14 @@ SDFR_API int32_t sdfr_goal_bake(const uint8_t* occ, int32_t nx, int32_t ny, int3
             if (host_counts[((k % 3u) * g.parts + p) * g.part_pitch]) done = false;
     }
     if (!done) return gfail(-7, "sdfr_goal_bake: not converged after %d sweeps", max_sweeps);
-    goal_reach_max<<<kReachBlocks, 256, 0, st>>>(g, L.vox);
+    goal_reach_max<<<kReachBlocks, 256, 0, st>>>(g);
     const double quant = (double)cell / 8.0;
     const float quant_f = (float)quant;
     const float inv_quant = 1.0f / quant_f;
-    const int wide = ((uintptr_t)grid_q & 7u) == 0 && ((uintptr_t)grid & 15u) == 0;
-    goal_quantise<<<init_blocks, 256, 0, st>>>(g.d, L.vox, g.ctl + kReach, (double)cell, inv_quant, quant_f, grid_q,
-                                               grid, wide);
+    const int wide = nx % 4 == 0 && ((uintptr_t)grid_q & 7u) == 0 && ((uintptr_t)grid & 15u) == 0;
+    const int64_t groups = (int64_t)((g.tx + 3) / 4) * g.ty * g.tz;
+    goal_quantise<<<(int)(groups > 65536 ? 65536 : groups), 256, 0, st>>>(g, (double)cell, inv_quant, quant_f, grid_q,
+                                                                           grid, wide);
     e = hipGetLastError();
     if (e == hipSuccess) e = hipMemcpyAsync(host_ctl, g.ctl, kCtl * 4, hipMemcpyDeviceToHost, st);
     if (e == hipSuccess) e = hipStreamSynchronize(st);

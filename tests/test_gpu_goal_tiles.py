@@ -62,3 +62,21 @@ def test_quantised_outputs_at_any_alignment(dev, shift):
     assert np.array_equal(q[shift:shift + n].cpu().numpy().view(np.uint16).reshape(shape), ref["grid_q"])
     assert np.array_equal(g[shift:shift + n].cpu().numpy().reshape(shape), ref["grid"])
     assert not q[shift + n:].any() and not g[shift + n:].any() and not q[:shift].any()
+
+
+@pytest.mark.parametrize("shape", [(24, 24, 40), (17, 23, 33), (8, 8, 4), (1, 1, 36)], ids=str)
+def test_tiles_without_a_free_voxel(dev, shape):
+    """Whole solid tiles, which are never queued: beside the seeds, under them, and in the way."""
+    occ = np.zeros(shape, np.uint8)
+    occ[:8, :8, 8:16] = 1                     # a solid tile inside the seed box
+    occ[8:16, 8:16, 16:24] = 1
+    occ[:8, 16:24, :8] = 1
+    zone = {"mins": [0.5, 0.5, 0.5], "maxs": [100.0, 30.0, 30.0]}
+    nz, ny, nx = shape
+    lo, hi = goalfield.seed_voxel_box(zone, np.zeros(3), 8.0, (nx, ny, nz))
+    print(f"case goal solid tiles {shape}", flush=True)
+    ref = ogoal.bake(occ, 8.0, lo, hi)
+    field = goalfield.goal_field_from_occupancy(occ, np.zeros(3), zone, 8.0, device=dev)
+    assert np.array_equal(field.grid_q.cpu().numpy().view(np.uint16), ref["grid_q"])
+    assert np.array_equal(field.grid.cpu().numpy(), ref["grid"])
+    assert field.bake_info["n_seed"] == ref["n_seed"]
