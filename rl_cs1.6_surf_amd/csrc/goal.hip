@@ -201,8 +201,9 @@ __device__ __forceinline__ void wave_sync() {
 // mark, slot: ~6 us). 256x256x128 voxels, 50 sweeps: 29 us a sweep with a block
 // of 512 threads and 26 LDS reads a voxel, 18 with a wave a tile, 16 with the
 // columns loaded straight to their lanes; a whole bake 1086 us with a queue
-// per XCD, 887 with the distances by tile. Also measured: flags per tile
-// instead of queues (no claims, but a static deal of tiles to waves: 28 us),
+// per XCD, 887 with the distances by tile, 840 with the halo's loads under a
+// branch and the pass down z as selects. Also measured: flags per tile instead
+// of queues (no claims, but a static deal of tiles to waves: 28 us a sweep),
 // reading a mark before its atomic (+2 us), no order along z (+2 us), queueing
 // only tiles whose halo copy would fall (20% fewer visits, each 3 us longer).
 __global__ __launch_bounds__(kThreads) void goal_sweep(GoalArgs a, const uint64_t* __restrict__ open_planes,
@@ -253,9 +254,14 @@ __global__ __launch_bounds__(kThreads) void goal_sweep(GoalArgs a, const uint64_
         // below and above; outside the grid nothing lowers a neighbour
         float* home = a.d + (int64_t)tile * kTileVox + lane * kT;
         const float* rim = a.d + (int64_t)tile * kTileVox + roff;
-        const float4 inf4 = make_float4(INFINITY, INFINITY, INFINITY, INFINITY);
         const float4 c0 = ((const float4*)home)[0], c1 = ((const float4*)home)[1];
-        const float4 r0 = on_ring ? ((const float4*)rim)[0] : inf4, r1 = on_ring ? ((const float4*)rim)[1] : inf4;
+        // (under a branch: as a choice of values the compiler chooses between
+        // addresses, one on the stack, and loads through the flat path)
+        float4 r0 = make_float4(INFINITY, INFINITY, INFINITY, INFINITY), r1 = r0;
+        if (on_ring) {
+            r0 = ((const float4*)rim)[0];
+            r1 = ((const float4*)rim)[1];
+        }
         float cb = INFINITY, ca = INFINITY, rb = INFINITY, ra = INFINITY;
         if (tz > 0) {   // uniform
             cb = home[kT - 1 - layer];
@@ -322,7 +328,10 @@ __global__ __launch_bounds__(kThreads) void goal_sweep(GoalArgs a, const uint64_
                 m[z] = __builtin_amdgcn_inverse_ballot_w64(open[z]) ? m[z] : INFINITY;
             }
 #pragma unroll
-            for (int z = kT - 2; z >= 0; --z) m[z] = __builtin_amdgcn_inverse_ballot_w64(open[z]) ? least(m[z], m[z + 1] + w1) : INFINITY;
+            for (int z = kT - 2; z >= 0; --z) {
+                const float down = least(m[z], m[z + 1] + w1);
+                m[z] = __builtin_amdgcn_inverse_ballot_w64(open[z]) ? down : INFINITY;
+            }
             bool lowered = false;
 #pragma unroll
             for (int z = 0; z < kT; ++z) {
