@@ -521,7 +521,7 @@ __global__ __launch_bounds__(256) void goal_sample(FieldArgs a, const void* __re
 // offset copies, samples, differences, atan2, degrees, remainder): four lanes
 // a position, one sample each, handed over by shuffles, so a position's 32
 // gathers are in flight together. 1500 host positions: 108 us a call before,
-// 47 now, most of it the copies there and back.
+// 42 now, most of it the copies there and back.
 template <int GRID, int POS>
 __global__ __launch_bounds__(256) void goal_yaw(FieldArgs a, const void* __restrict__ pos, int64_t pos_stride,
                                                 int64_t n, float* __restrict__ out) {

@@ -159,7 +159,7 @@ class GoalField:
     def _launch(self, entry, p, code, stride, n, out):
         lib = _sdfr.load()
         nz, ny, nx = self._grid.shape
-        rc = getattr(lib, entry)(self._grid.data_ptr(), self._kind, self.quant, nx, ny, nz, self._mins_c,
+        rc = getattr(lib, entry)(self._grid.data_ptr(), self._kind, float(self.quant), nx, ny, nz, self._mins_c,
                                  self.cell, self.reach_max, p.data_ptr(), code, stride, n,
                                  out.data_ptr(), vision._current_stream(self.device))
         if rc != 0:
