@@ -108,18 +108,6 @@ static_assert(kOrderBuckets % 256 == 0, "the sort blocks' 256 threads take 16 bu
 // (1.0-1.2).
 constexpr float kOrderLookahead = 1.2f;
 constexpr float kOrderLookaheadSpilled = 3.0f;
-// Renders of at least kOrderTraceTiles tiles on those grids key a unit by where
-// its centre ray is after kOrderTraceSteps samples, at most the lookahead out:
-// a ray that ends sooner says better where its tile's samples lie. 2048 envs: a
-// closed 1 GiB fp32 map 2.048 -> 1.888 ms, the open 1 GiB track 1.808 -> 1.787,
-// a 1.3 GB fp16 map 1.101 -> 1.103 (its march gains 12 us, keying costs 13).
-// Fewer samples stop short of where the ray looks (8: 1.927 / 1.792 / 1.108 ms;
-// 4 with the older split 2.097 / 1.942 / 1.165), 13: 1.885 / 1.805 / 1.102.
-// Smaller renders would wait longer for the ten dependent misses than they
-// gain (the track at 512 and 1024 envs 1.5-3% slower), and on cache-resident
-// grids the plain key is the better one (32 MiB fp32: 366 against 392 us).
-constexpr int kOrderTraceSteps = 10;
-constexpr int64_t kOrderTraceTiles = 1 << 18;
 // Renders of fewer tiles skip the sort by default: its two launches cost
 // ~9 us, more than it saves below ~512 envs of 128x64.
 constexpr int64_t kOrderMinTiles = 1 << 16;
@@ -459,12 +447,11 @@ __device__ __forceinline__ int2 tile_corner(const MarchArgs& a, int t) {
 }
 
 // -------------------------------------------------------------- ray setup --
-// The grid value at a point, for stores and layouts known at run time. At an
-// eye it is what every ray of the env reads at its first step: at t = 0 the
+// The grid value every ray of an env reads at its first step: at t = 0 the
 // sample point e + d*0 is the eye itself for every direction (e + (+-0) = e
 // up to the sign of a zero, which the index formula maps to the same voxel),
 // so the whole env shares one first sample. 0 when there is no grid.
-__device__ __forceinline__ float point_sample(const MarchArgs& a, float ex, float ey, float ez) {
+__device__ __forceinline__ float eye_sample(const MarchArgs& a, float ex, float ey, float ez) {
     if (!a.grid) return 0.0f;
     const int ix = (int)__builtin_amdgcn_fmed3f((ex - a.mnx) * a.inv_cell, 0.0f, a.fnx1);
     const int iy = (int)__builtin_amdgcn_fmed3f((ey - a.mny) * a.inv_cell, 0.0f, a.fny1);
@@ -507,7 +494,7 @@ __device__ __forceinline__ float2 table_entry(const MarchArgs& a, int n, int e) 
     if (e == 0) return make_float2(a.origin[n * a.origin_stride + 0], a.origin[n * a.origin_stride + 1]);
     if (e == 1) {
         const float ez = eye_z(a, n);
-        return make_float2(ez, point_sample(a, a.origin[n * a.origin_stride + 0],
+        return make_float2(ez, eye_sample(a, a.origin[n * a.origin_stride + 0],
                                           a.origin[n * a.origin_stride + 1], ez));
     }
     if (a.camera != SDFR_CAM_PINHOLE) return make_float2(0.0f, 0.0f);
@@ -635,10 +622,9 @@ __device__ __forceinline__ void fill_axis_tables(const MarchArgs& a, uint32_t* s
 // consecutive tiles: the upper or lower half of a quad, or a whole quad, a
 // 32-pixel-wide block of one env, so the waves of a workgroup march similar
 // rays and end together); each unit is keyed by
-// where its centre ray is after `lookahead` units of distance (1.2 x the near
-// range, 3 x on grids beyond the Infinity Cache, where large renders stop
-// sooner if the ray does): the cell (of a grid of at most 16^3 cells over the
-// voxel grid) holding that point, numbered along a Morton curve. A counting sort by
+// where its centre ray is after `lookahead` units of distance (1.2 x the
+// near range): the cell (of a grid of at most 16^3 cells over the voxel
+// grid) holding that point, numbered along a Morton curve. A counting sort by
 // key gives the permutation of units; the march then deals chunks of the
 // sorted list to the XCDs (xcd_chunked_block), so at any time each XCD's L2
 // serves rays that look at one part of the map. Results do not depend on the
@@ -657,16 +643,11 @@ __device__ __forceinline__ uint32_t spread_bits4(uint32_t v) {
     return (v & 1u) | ((v & 2u) << 2) | ((v & 4u) << 4) | ((v & 8u) << 6);
 }
 
-// The centre ray of a unit, in fast fp32 arithmetic (the ray tables are
-// written by the same launch); it only orders the tiles, so its precision
-// does not touch the results.
-struct UnitRay {
-    float ex, ey, ez;
-    float3 d;
-};
-
+// The key of a unit, from its centre ray, in fast fp32 arithmetic (the ray
+// tables are written by the same launch); the key only orders the tiles, so
+// its precision does not touch the results.
 template <int CAMERA>
-__device__ __forceinline__ UnitRay unit_ray(const MarchArgs& a, int64_t unit) {
+__device__ __forceinline__ uint32_t tile_order_key(const MarchArgs& a, int64_t unit) {
     // the unit's centre pixel: a unit is two tiles side by side (one quad's
     // upper or lower half) or a whole quad, and starts at a tile with q = 0
     // or 2, so its centre is kTileW right of its first tile's corner and half
@@ -691,15 +672,13 @@ __device__ __forceinline__ UnitRay unit_ray(const MarchArgs& a, int64_t unit) {
         row = make_float2(__sinf(p), __cosf(p));
         col = make_float2(__sinf(y), __cosf(y));
     }
-    return UnitRay{a.origin[n * a.origin_stride + 0], a.origin[n * a.origin_stride + 1], eye_z(a, n),
-                   ray_dir<CAMERA>(row, col, psc, ysc)};
-}
-
-// The key of a unit: the cell of its centre ray's point at distance L.
-__device__ __forceinline__ uint32_t order_key_at(const MarchArgs& a, const UnitRay& u, float L) {
-    const int ix = (int)__builtin_amdgcn_fmed3f((u.ex + u.d.x * L - a.mnx) * a.inv_cell, 0.0f, a.fnx1);
-    const int iy = (int)__builtin_amdgcn_fmed3f((u.ey + u.d.y * L - a.mny) * a.inv_cell, 0.0f, a.fny1);
-    const int iz = (int)__builtin_amdgcn_fmed3f((u.ez + u.d.z * L - a.mnz) * a.inv_cell, 0.0f, a.fnz1);
+    const float3 d = ray_dir<CAMERA>(row, col, psc, ysc);
+    const float L = a.lookahead;
+    const float ex = a.origin[n * a.origin_stride + 0], ey = a.origin[n * a.origin_stride + 1];
+    const float ez = eye_z(a, n);
+    const int ix = (int)__builtin_amdgcn_fmed3f((ex + d.x * L - a.mnx) * a.inv_cell, 0.0f, a.fnx1);
+    const int iy = (int)__builtin_amdgcn_fmed3f((ey + d.y * L - a.mny) * a.inv_cell, 0.0f, a.fny1);
+    const int iz = (int)__builtin_amdgcn_fmed3f((ez + d.z * L - a.mnz) * a.inv_cell, 0.0f, a.fnz1);
     return spread_bits4((uint32_t)ix >> a.order_shift) |
            (spread_bits4((uint32_t)iy >> a.order_shift) << 1) |
            (spread_bits4((uint32_t)iz >> a.order_shift) << 2);
@@ -714,11 +693,7 @@ constexpr int kOrderChunk = 1024;
 // entry per thread. The sort blocks run ~4x longer than a table block, so
 // they come first: dispatched last, they started only once the table blocks
 // had been dealt out (at 8192 envs 11 us into the launch) and set its end.
-// PER: units a thread keys; with TRACE it marches their centre rays first. That
-// is ten dependent misses, bound by the misses a CU keeps in flight, so a
-// thread then keys one unit, which spreads 2048 envs over 512 blocks (four a
-// thread, stepped together: 128 blocks, 10 us longer).
-template <int CAMERA, int PER, bool TRACE>
+template <int CAMERA>
 __global__ __launch_bounds__(256) void ray_setup(MarchArgs a, int sort_blocks) {
     if ((int)blockIdx.x >= sort_blocks) {
         const int64_t i = (int64_t)(blockIdx.x - sort_blocks) * blockDim.x + threadIdx.x;
@@ -728,11 +703,11 @@ __global__ __launch_bounds__(256) void ray_setup(MarchArgs a, int sort_blocks) {
         a.rt[i] = table_entry(a, n, e);
         return;
     }
-    constexpr int kPer = PER;
+    constexpr int kPer = kOrderChunk / 256;
     __shared__ uint32_t h[kOrderBuckets];
     for (int i = threadIdx.x; i < kOrderBuckets; i += blockDim.x) h[i] = 0u;
     __syncthreads();
-    const int64_t u0 = (int64_t)blockIdx.x * (256 * PER);
+    const int64_t u0 = (int64_t)blockIdx.x * kOrderChunk;
     uint32_t key[kPer], rank[kPer];
 #pragma unroll
     for (int j = 0; j < kPer; ++j) {
@@ -740,18 +715,7 @@ __global__ __launch_bounds__(256) void ray_setup(MarchArgs a, int sort_blocks) {
         key[j] = 0u;
         rank[j] = 0u;
         if (u < a.order_units) {
-            const UnitRay ray = unit_ray<CAMERA>(a, u);
-            float t = a.lookahead;
-            if constexpr (TRACE) {
-                t = 0.0f;
-                for (int k = 0; k < kOrderTraceSteps; ++k) {
-                    const float sd = point_sample(a, ray.ex + ray.d.x * t, ray.ey + ray.d.y * t, ray.ez + ray.d.z * t);
-                    if (!(sd > a.hit_eps && t < a.lookahead)) break;
-                    t += fmaxf(sd * 0.9f, a.min_step);
-                }
-                t = fminf(t, a.lookahead);
-            }
-            key[j] = order_key_at(a, ray, t);
+            key[j] = tile_order_key<CAMERA>(a, u);
             rank[j] = atomicAdd(&h[key[j]], 1u);
         }
     }
@@ -1736,11 +1700,9 @@ int32_t render_impl(const char* fn, const SdfrGrid* grid, const SdfrCam* cam, co
     const int64_t entries = (int64_t)poses->n_envs * a.rt_stride;
     const int64_t table_blocks = (entries + 255) / 256;
     const int64_t sort_blocks = a.perm ? (a.order_units + kOrderChunk - 1) / kOrderChunk : 0;
-    const bool trace = a.perm && grid->store_bytes > kCacheResidentBytes && a.total_tiles >= kOrderTraceTiles;
-    const int64_t key_blocks = trace ? (a.order_units + 255) / 256 : sort_blocks;
-    if (table_blocks + key_blocks > 0x7fffffff)
+    if (table_blocks + sort_blocks > 0x7fffffff)
         return fail(-2, "%s: too many envs (%lld ray-setup blocks)", fn,
-                    (long long)(table_blocks + key_blocks));
+                    (long long)(table_blocks + sort_blocks));
 
     hipStream_t st = (hipStream_t)stream;
     hipError_t e = hipGetLastError();   // an earlier, unrelated error must not be taken for ours
@@ -1753,12 +1715,10 @@ int32_t render_impl(const char* fn, const SdfrGrid* grid, const SdfrCam* cam, co
         grid->hist_dirty = false;
     }
     if (!a.inline_setup) {
-        constexpr int kPer = kOrderChunk / 256;
-        const bool pinhole = cam->camera == SDFR_CAM_PINHOLE;
-        auto* setup = trace ? (pinhole ? ray_setup<SDFR_CAM_PINHOLE, 1, true> : ray_setup<SDFR_CAM_EQUIANGULAR, 1, true>)
-                            : (pinhole ? ray_setup<SDFR_CAM_PINHOLE, kPer, false>
-                                       : ray_setup<SDFR_CAM_EQUIANGULAR, kPer, false>);
-        setup<<<(int)(table_blocks + key_blocks), 256, 0, st>>>(a, (int)key_blocks);
+        if (cam->camera == SDFR_CAM_PINHOLE)
+            ray_setup<SDFR_CAM_PINHOLE><<<(int)(table_blocks + sort_blocks), 256, 0, st>>>(a, (int)sort_blocks);
+        else
+            ray_setup<SDFR_CAM_EQUIANGULAR><<<(int)(table_blocks + sort_blocks), 256, 0, st>>>(a, (int)sort_blocks);
         e = hipGetLastError();
         if (e != hipSuccess) return fail(-4, "%s: ray setup launch failed: %s", fn, hipGetErrorString(e));
     }
