@@ -592,15 +592,18 @@ int tile_words(int n, int cell_bytes, int64_t lds_limit, size_t* lds) {
 }
 
 template <typename V, int OUT, bool EXACT>
-hipError_t launch_tile(PassArgs a, int tw, size_t lds, int outer, hipStream_t st) {
+hipError_t launch_tile(PassArgs a, int tw, size_t lds, int lds_limit, int outer, hipStream_t st) {
     a.blks = (a.n + kBlk - 1) / kBlk;
     const int vox = tw * Word<V>::kVox;
     a.tiles = (a.nx + vox - 1) / vox;
     a.blocks = (int64_t)a.tiles * outer;
     auto* k = tw == 32 ? edt_tile<V, 32, OUT, EXACT> : tw == 16 ? edt_tile<V, 16, OUT, EXACT> : edt_tile<V, 8, OUT, EXACT>;
     if (lds > (64 << 10)) {
+        // the attribute belongs to the process: every call sets the device's
+        // limit, not its own size, so that no thread's launch meets a smaller
+        // size that another thread has set for its grid
         const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(k),
-                                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+                                                 hipFuncAttributeMaxDynamicSharedMemorySize, lds_limit);
         if (e != hipSuccess) return e;
     }
     const int items = a.blks * tw;   // one kBlk-output search each
@@ -611,9 +614,12 @@ hipError_t launch_tile(PassArgs a, int tw, size_t lds, int outer, hipStream_t st
 }
 
 template <typename V>
-hipError_t launch_z(const PassArgs& a, bool f32, bool exact, int tw, size_t lds, hipStream_t st) {
-    if (f32) return exact ? launch_tile<V, kF32, true>(a, tw, lds, a.ny, st) : launch_tile<V, kF32, false>(a, tw, lds, a.ny, st);
-    return exact ? launch_tile<V, kF16, true>(a, tw, lds, a.ny, st) : launch_tile<V, kF16, false>(a, tw, lds, a.ny, st);
+hipError_t launch_z(const PassArgs& a, bool f32, bool exact, int tw, size_t lds, int limit, hipStream_t st) {
+    if (f32)
+        return exact ? launch_tile<V, kF32, true>(a, tw, lds, limit, a.ny, st)
+                     : launch_tile<V, kF32, false>(a, tw, lds, limit, a.ny, st);
+    return exact ? launch_tile<V, kF16, true>(a, tw, lds, limit, a.ny, st)
+                 : launch_tile<V, kF16, false>(a, tw, lds, limit, a.ny, st);
 }
 
 // Bytes hold every distance along x that can matter (255^2 >= z_cap), and 16
@@ -717,13 +723,13 @@ SDFR_API int32_t sdfr_edt(const uint8_t* occ, int32_t nx, int32_t ny, int32_t nz
         p.n = ny;
         p.out = p.plane;
         if (e == hipSuccess)
-            e = packed ? launch_tile<u16x2, kPlane, true>(p, tw_y, lds_y, nz, st)
-                       : launch_tile<uint32_t, kPlane, true>(p, tw_y, lds_y, nz, st);
+            e = packed ? launch_tile<u16x2, kPlane, true>(p, tw_y, lds_y, lds_limit, nz, st)
+                       : launch_tile<uint32_t, kPlane, true>(p, tw_y, lds_y, lds_limit, nz, st);
         p.n = nz;
         p.out = out;
         if (e == hipSuccess)
-            e = packed ? launch_z<u16x2>(p, fout != nullptr, exact, tw_z, lds_z, st)
-                       : launch_z<uint32_t>(p, fout != nullptr, exact, tw_z, lds_z, st);
+            e = packed ? launch_z<u16x2>(p, fout != nullptr, exact, tw_z, lds_z, lds_limit, st)
+                       : launch_z<uint32_t>(p, fout != nullptr, exact, tw_z, lds_z, lds_limit, st);
         if (e != hipSuccess) return efail(-4, "sdfr_edt: launch failed: %s", hipGetErrorString(e));
         return 0;
     }
