@@ -247,11 +247,11 @@ __global__ __launch_bounds__(256) void edt_slabs(const int32_t* __restrict__ f, 
 //     sqrt(z_cap); for nz <= 509 the squares fit 16 bits (two voxels a
 //     register, v_pk_add_u16 saturating and v_pk_min_u16) and the distances
 //     along x a byte.
-//   * A thread takes kBlk consecutive outputs of a line (two lines when
+//   * A thread takes BLK consecutive outputs of a line (two lines when
 //     packed) in registers and reads each candidate once for all of them.
-//   * Candidates come in chunks of kBlk rows, nearest first, on both sides,
+//   * Candidates come in chunks of BLK rows, nearest first, on both sides,
 //     until even a zero in the next chunk could not win (its nearest row is
-//     kBlk(c - 1) + 1 away); a chunk whose smallest value (kept per chunk and
+//     BLK(c - 1) + 1 away); a chunk whose smallest value (kept per chunk and
 //     line) cannot win at that distance either is skipped. Neighbouring lines
 //     agree about both, so on the scenes measured a wave searches ~4 of a
 //     line's 128 chunks.
@@ -267,7 +267,8 @@ __global__ __launch_bounds__(256) void edt_slabs(const int32_t* __restrict__ f, 
 // (749 against 930 us), and lose in the z pass (741 against 622).
 typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
 
-constexpr int kBlk = 8;
+constexpr int kBlk = 8;       // outputs a thread takes and rows a chunk holds, ...
+constexpr int kSmallBlk = 2;  // ... and in small grids (small_grid)
 constexpr int kThreadsY = 1024, kThreadsZ = 512;
 
 template <typename V> struct Word;
@@ -428,9 +429,9 @@ struct PassArgs {
 
 // Row of a tile in LDS: a row's gap after each block of rows, so that the
 // blocks a wave works on lie on different banks.
-template <int TW>
+template <int TW, int BLK>
 __device__ __forceinline__ int tile_row(int row) {
-    return (row + row / kBlk) * TW;
+    return (row + row / BLK) * TW;
 }
 
 // What a pass writes: the plane of squares (y pass), or the distances.
@@ -464,7 +465,7 @@ __device__ __forceinline__ void put_distances(const PassArgs& a, O* o, V v, int 
     }
 }
 
-template <typename V, int TW, int OUT, bool EXACT>
+template <typename V, int TW, int OUT, bool EXACT, int BLK>
 __global__ __launch_bounds__(OUT == kPlane ? kThreadsY : kThreadsZ) void edt_tile(PassArgs a) {
     constexpr bool Z = OUT != kPlane;
     using W = Word<V>;
@@ -473,7 +474,7 @@ __global__ __launch_bounds__(OUT == kPlane ? kThreadsY : kThreadsZ) void edt_til
     using T = typename C::T;
     extern __shared__ uint32_t smem[];
     T* s = (T*)smem;                                                  // the tile's lines
-    T* cmin = s + (size_t)tile_row<TW>(a.blks * kBlk);                // smallest of each chunk
+    T* cmin = s + (size_t)tile_row<TW, BLK>(a.blks * BLK);                // smallest of each chunk
     const int64_t tile = xcd_tile(blockIdx.x, a.blocks);
     const int outer = (int)(tile / a.tiles);             // z (y pass) or y (z pass)
     const int xt = (int)(tile - (int64_t)outer * a.tiles) * TW * W::kVox;
@@ -485,12 +486,12 @@ __global__ __launch_bounds__(OUT == kPlane ? kThreadsY : kThreadsZ) void edt_til
     if constexpr (Z) {
         const P* p = (const P*)a.plane + (int64_t)outer * a.pitch + x;
         const int64_t step = (int64_t)a.ny * a.pitch;
-        for (int row = row0; row < a.blks * kBlk; row += rows)
-            s[tile_row<TW>(row) + col] = row < n && x < a.nx ? C::shut(*(const V*)(p + row * step)) : C::shut(C::far());
+        for (int row = row0; row < a.blks * BLK; row += rows)
+            s[tile_row<TW, BLK>(row) + col] = row < n && x < a.nx ? C::shut(*(const V*)(p + row * step)) : C::shut(C::far());
     } else {
         const uint2* p = a.bits + ((int64_t)outer * a.words + (x >> 5)) * n;
         const int i = x & 31;
-        for (int row = row0; row < a.blks * kBlk; row += rows) {
+        for (int row = row0; row < a.blks * BLK; row += rows) {
             V v = C::far();
             if (row < n && x < a.nx) {
                 const uint2 b = p[row];
@@ -502,27 +503,27 @@ __global__ __launch_bounds__(OUT == kPlane ? kThreadsY : kThreadsZ) void edt_til
                     v = g0 * g0;
                 }
             }
-            s[tile_row<TW>(row) + col] = C::shut(v);
+            s[tile_row<TW, BLK>(row) + col] = C::shut(v);
         }
     }
     __syncthreads();
     for (int k = row0; k < a.blks; k += rows) {
-        const T* p = s + tile_row<TW>(k * kBlk) + col;
+        const T* p = s + tile_row<TW, BLK>(k * BLK) + col;
         V m = C::open(p[0]);
 #pragma unroll
-        for (int r = 1; r < kBlk; ++r) m = __builtin_elementwise_min(m, C::open(p[r * TW]));
+        for (int r = 1; r < BLK; ++r) m = __builtin_elementwise_min(m, C::open(p[r * TW]));
         cmin[k * TW + col] = C::shut(m);
     }
     __syncthreads();
     if (x >= a.nx) return;
     const uint32_t cap = Z ? W::kMax : min((uint32_t)(outer + 1) * (uint32_t)(a.nz - outer), W::kMax);   // z_cap
     for (int blk = row0; blk < a.blks; blk += rows) {
-        const int q0 = blk * kBlk;
-        const T* own = s + tile_row<TW>(q0) + col;
-        V best[kBlk];
+        const int q0 = blk * BLK;
+        const T* own = s + tile_row<TW, BLK>(q0) + col;
+        V best[BLK];
         V most = W::splat(0u);
 #pragma unroll
-        for (int r = 0; r < kBlk; ++r) {
+        for (int r = 0; r < BLK; ++r) {
             // the value above, and the solid rows at -1 and n; rows past the
             // end take part in nothing
             const int e = min(q0 + r + 1, n - q0 - r);
@@ -533,20 +534,20 @@ __global__ __launch_bounds__(OUT == kPlane ? kThreadsY : kThreadsZ) void edt_til
         // the chunk of rows at p, row j at distance d(j, r) from output r
         auto take = [&](const T* p, auto square) {
 #pragma unroll
-            for (int j = 0; j < kBlk; ++j) {
+            for (int j = 0; j < BLK; ++j) {
                 const V v = C::value(C::open(p[j * TW]));
 #pragma unroll
-                for (int r = 0; r < kBlk; ++r)
+                for (int r = 0; r < BLK; ++r)
                     best[r] = __builtin_elementwise_min(best[r], W::add(v, square(j, r)));
             }
             most = best[0];
 #pragma unroll
-            for (int r = 1; r < kBlk; ++r) most = __builtin_elementwise_max(most, best[r]);
+            for (int r = 1; r < BLK; ++r) most = __builtin_elementwise_max(most, best[r]);
         };
         if (W::any_less(C::value(C::open(cmin[blk * TW + col])), most))
             take(own, [](int j, int r) { return W::splat((uint32_t)((j - r) * (j - r))); });
         for (int c = 1;; ++c) {
-            const uint32_t near = (uint32_t)(kBlk * (c - 1) + 1);   // of the chunk's nearest row
+            const uint32_t near = (uint32_t)(BLK * (c - 1) + 1);   // of the chunk's nearest row
             const V near2 = W::splat(min(near * near, W::kMax));
             const bool go = W::any_less(near2, most);
             if (!__any(go)) break;
@@ -554,21 +555,21 @@ __global__ __launch_bounds__(OUT == kPlane ? kThreadsY : kThreadsZ) void edt_til
             const bool has_up = up < a.blks, has_down = down >= 0;
             if (!__any(has_up || has_down)) break;
             // row j is near + j beyond the last output or before the first
-            V sq[2 * kBlk - 1];
+            V sq[2 * BLK - 1];
 #pragma unroll
-            for (int k = 0; k < 2 * kBlk - 1; ++k)
+            for (int k = 0; k < 2 * BLK - 1; ++k)
                 sq[k] = W::splat(min((near + (uint32_t)k) * (near + (uint32_t)k), W::kMax));
             if (go && has_up && W::any_less(W::add(C::value(C::open(cmin[up * TW + col])), near2), most))
-                take(s + tile_row<TW>(up * kBlk) + col, [&](int j, int r) { return sq[j + kBlk - 1 - r]; });
+                take(s + tile_row<TW, BLK>(up * BLK) + col, [&](int j, int r) { return sq[j + BLK - 1 - r]; });
             if (go && has_down && W::any_less(W::add(C::value(C::open(cmin[down * TW + col])), near2), most))
-                take(s + tile_row<TW>(down * kBlk) + col, [&](int j, int r) { return sq[kBlk - 1 - j + r]; });
+                take(s + tile_row<TW, BLK>(down * BLK) + col, [&](int j, int r) { return sq[BLK - 1 - j + r]; });
         }
         const int64_t step = Z ? (int64_t)a.ny * a.nx : a.pitch;
         const int64_t first = Z ? ((int64_t)q0 * a.ny + outer) * a.nx + x : ((int64_t)outer * n + q0) * a.pitch + x;
         using O = typename std::conditional<OUT == kPlane, P, typename std::conditional<OUT == kF32, float, __half>::type>::type;
         O* o = (O*)a.out + first;
 #pragma unroll
-        for (int r = 0; r < kBlk; ++r) {
+        for (int r = 0; r < BLK; ++r) {
             if (q0 + r < n) {
                 if constexpr (!Z) *(V*)(o + r * step) = best[r];
                 else put_distances<V, O, EXACT>(a, o + r * step, best[r], x);
@@ -577,12 +578,32 @@ __global__ __launch_bounds__(OUT == kPlane ? kThreadsY : kThreadsZ) void edt_til
     }
 }
 
+// Whether a grid has too few rows, and too short searches (the z bound), to
+// fill the GPU with kBlk outputs a thread. What bounds its passes is one
+// thread's chain: its loads in turn, and searches unrolled into more code than
+// they run. kSmallBlk shortens both, and edt_pack takes fewer rows a block.
+// The three launches in a graph, us, 1% of the voxels solid (none in the last
+// three rows), with a wave a row and a search per output / kBlk / kSmallBlk and
+// the short blocks of edt_pack:
+//   40x40x16 voxels 11.3 / 15.9 / 11.7     200x40x16 13.5 / 19.5 / 13.1
+//   300x60x16       17.0 / 21.2 / 13.7     900x40x16 26.3 / 25.6 / 15.3
+//   64x64x64        28.7 / 18.3 / 18.4 (the last on this side of both lines)
+//   40x40x128       39.5 / 16.4 / 24.5
+//   300x300x16       117 / 25.7 / 28.3
+bool small_grid(int nx, int ny, int nz) {
+    const int64_t rows = (int64_t)ny * nz;
+    return rows <= 4096 && rows * nx * nz <= 1 << 24;
+}
+
 // Words a tile is wide for lines of n, and its LDS bytes; 0 where even the
-// narrowest does not fit the workgroup's LDS.
-int tile_words(int n, int cell_bytes, int64_t lds_limit, size_t* lds) {
-    const int64_t blks = (n + kBlk - 1) / kBlk;
+// narrowest does not fit the workgroup's LDS. Rows `across` words long get no
+// wider tile than covers them: its other lanes would work on padding (1x1500x40
+// voxels 48 us 32 words wide, 21 us 8 wide; 16x200x600 46 and 30).
+int tile_words(int n, int across, int blk, int cell_bytes, int64_t lds_limit, size_t* lds) {
+    const int64_t blks = (n + blk - 1) / blk;
     for (int tw : {32, 16, 8}) {
-        const int64_t bytes = blks * (kBlk + 2) * tw * cell_bytes;   // rows, gap and minimum
+        if (tw > 8 && tw / 2 >= across) continue;
+        const int64_t bytes = blks * (blk + 2) * tw * cell_bytes;   // rows, gap and minimum
         if (bytes <= lds_limit) {
             *lds = (size_t)bytes;
             return tw;
@@ -591,35 +612,48 @@ int tile_words(int n, int cell_bytes, int64_t lds_limit, size_t* lds) {
     return 0;
 }
 
-template <typename V, int OUT, bool EXACT>
-hipError_t launch_tile(PassArgs a, int tw, size_t lds, int lds_limit, int outer, hipStream_t st) {
-    a.blks = (a.n + kBlk - 1) / kBlk;
+// A pass's tiles: `blk` outputs a thread, `tw` words wide, `lds` bytes of the
+// device's `limit`.
+struct TilePlan {
+    int blk, tw, limit;
+    size_t lds;
+};
+
+template <typename V, int OUT, bool EXACT, int BLK>
+hipError_t launch_tile(PassArgs a, const TilePlan& t, int outer, hipStream_t st) {
+    const int tw = t.tw;
+    a.blks = (a.n + BLK - 1) / BLK;
     const int vox = tw * Word<V>::kVox;
     a.tiles = (a.nx + vox - 1) / vox;
     a.blocks = (int64_t)a.tiles * outer;
-    auto* k = tw == 32 ? edt_tile<V, 32, OUT, EXACT> : tw == 16 ? edt_tile<V, 16, OUT, EXACT> : edt_tile<V, 8, OUT, EXACT>;
-    if (lds > (64 << 10)) {
+    auto* k = tw == 32   ? edt_tile<V, 32, OUT, EXACT, BLK>
+              : tw == 16 ? edt_tile<V, 16, OUT, EXACT, BLK>
+                         : edt_tile<V, 8, OUT, EXACT, BLK>;
+    if (t.lds > (64 << 10)) {
         // the attribute belongs to the process: every call sets the device's
         // limit, not its own size, so that no thread's launch meets a smaller
         // size that another thread has set for its grid
         const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(k),
-                                                 hipFuncAttributeMaxDynamicSharedMemorySize, lds_limit);
+                                                 hipFuncAttributeMaxDynamicSharedMemorySize, t.limit);
         if (e != hipSuccess) return e;
     }
-    const int items = a.blks * tw;   // one kBlk-output search each
+    const int items = a.blks * tw;   // one BLK-output search each
     const int most = OUT == kPlane ? kThreadsY : kThreadsZ;
     const int threads = items >= most ? most : (items + 63) & ~63;
-    k<<<(unsigned)a.blocks, threads, lds, st>>>(a);
+    k<<<(unsigned)a.blocks, threads, t.lds, st>>>(a);
     return hipGetLastError();
 }
 
+template <typename V, int OUT, bool EXACT>
+hipError_t launch_tile(const PassArgs& a, const TilePlan& t, int outer, hipStream_t st) {
+    return t.blk == kBlk ? launch_tile<V, OUT, EXACT, kBlk>(a, t, outer, st)
+                         : launch_tile<V, OUT, EXACT, kSmallBlk>(a, t, outer, st);
+}
+
 template <typename V>
-hipError_t launch_z(const PassArgs& a, bool f32, bool exact, int tw, size_t lds, int limit, hipStream_t st) {
-    if (f32)
-        return exact ? launch_tile<V, kF32, true>(a, tw, lds, limit, a.ny, st)
-                     : launch_tile<V, kF32, false>(a, tw, lds, limit, a.ny, st);
-    return exact ? launch_tile<V, kF16, true>(a, tw, lds, limit, a.ny, st)
-                 : launch_tile<V, kF16, false>(a, tw, lds, limit, a.ny, st);
+hipError_t launch_z(const PassArgs& a, bool f32, bool exact, const TilePlan& t, hipStream_t st) {
+    if (f32) return exact ? launch_tile<V, kF32, true>(a, t, a.ny, st) : launch_tile<V, kF32, false>(a, t, a.ny, st);
+    return exact ? launch_tile<V, kF16, true>(a, t, a.ny, st) : launch_tile<V, kF16, false>(a, t, a.ny, st);
 }
 
 // Bytes hold every distance along x that can matter (255^2 >= z_cap), and 16
@@ -697,9 +731,18 @@ SDFR_API int32_t sdfr_edt(const uint8_t* occ, int32_t nx, int32_t ny, int32_t nz
         hipDeviceGetAttribute(&lds_limit, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess)
         lds_limit = 64 << 10;
     const bool packed = nz <= kPackedMaxNz;
-    size_t lds_y = 0, lds_z = 0;
-    const int tw_y = tile_words(ny, packed ? 2 : 4, lds_limit, &lds_y), tw_z = tile_words(nz, 4, lds_limit, &lds_z);
-    if (tw_y && tw_z) {
+    const bool small = small_grid(nx, ny, nz);
+    TilePlan ty, tz;
+    ty.limit = tz.limit = lds_limit;
+    const int across = packed ? (nx + 1) / 2 : nx;
+    for (int blk : {kSmallBlk, kBlk}) {   // (1.6 times the LDS: a line that does not fit so may with kBlk)
+        if (blk == kSmallBlk && !small) continue;
+        ty.blk = tz.blk = blk;
+        ty.tw = tile_words(ny, across, blk, packed ? 2 : 4, lds_limit, &ty.lds);
+        tz.tw = tile_words(nz, across, blk, 4, lds_limit, &tz.lds);
+        if (ty.tw && tz.tw) break;
+    }
+    if (ty.tw && tz.tw) {
         // the bits, then the plane of squares (edt_scratch_bytes holds both)
         PassArgs p;
         memset(&p, 0, sizeof p);
@@ -714,7 +757,7 @@ SDFR_API int32_t sdfr_edt(const uint8_t* occ, int32_t nx, int32_t ny, int32_t nz
         p.cell2f = (float)cell2;
         const bool exact = exact_in_f32(cell2, nx, ny, nz);
         p.wide = nx % 2 == 0 && ((uintptr_t)out & (fout ? 7u : 3u)) == 0;
-        int R = 512 / p.words;
+        int R = (small ? 128 : 512) / p.words;   // 128: a half word a thread, in one round
         R = R < 1 ? 1 : R > 32 ? 32 : R;
         const int wide_in = nx % 16 == 0 && ((uintptr_t)occ & 15u) == 0;
         edt_pack<<<(unsigned)((rows + R - 1) / R), 256, (size_t)R * (p.words + 1) * 4, st>>>(
@@ -723,13 +766,13 @@ SDFR_API int32_t sdfr_edt(const uint8_t* occ, int32_t nx, int32_t ny, int32_t nz
         p.n = ny;
         p.out = p.plane;
         if (e == hipSuccess)
-            e = packed ? launch_tile<u16x2, kPlane, true>(p, tw_y, lds_y, lds_limit, nz, st)
-                       : launch_tile<uint32_t, kPlane, true>(p, tw_y, lds_y, lds_limit, nz, st);
+            e = packed ? launch_tile<u16x2, kPlane, true>(p, ty, nz, st)
+                       : launch_tile<uint32_t, kPlane, true>(p, ty, nz, st);
         p.n = nz;
         p.out = out;
         if (e == hipSuccess)
-            e = packed ? launch_z<u16x2>(p, fout != nullptr, exact, tw_z, lds_z, lds_limit, st)
-                       : launch_z<uint32_t>(p, fout != nullptr, exact, tw_z, lds_z, lds_limit, st);
+            e = packed ? launch_z<u16x2>(p, fout != nullptr, exact, tz, st)
+                       : launch_z<uint32_t>(p, fout != nullptr, exact, tz, st);
         if (e != hipSuccess) return efail(-4, "sdfr_edt: launch failed: %s", hipGetErrorString(e));
         return 0;
     }

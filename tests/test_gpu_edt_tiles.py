@@ -21,6 +21,13 @@ pytestmark = pytest.mark.gpu
 SHAPES = [(7, 8, 31), (8, 9, 32), (9, 7, 33), (17, 16, 1), (15, 33, 63), (24, 25, 130),
           (509, 40, 21), (510, 40, 21), (509, 530, 3), (4, 1030, 6), (3, 3000, 5), (2, 5000, 7),
           (1500, 5, 6), (2100, 4, 3), (3, 2, 1500), (4500, 3, 5), (2, 9000, 3)]
+# past 4096 rows, or 2^24 voxels times planes, a block is 8 rows and not 2: either side of both
+# lines, and the edges above past them; rows around the widths that 8, 16 and 32 words cover, one
+# and two voxels a word; z lines that fit the LDS with blocks of 8 only
+SHAPES += [(64, 64, 64), (64, 64, 65), (65, 64, 33), (7, 590, 31), (8, 513, 32), (9, 456, 34), (17, 241, 97),
+           (64, 65, 1), (129, 33, 16), (129, 33, 17), (129, 33, 32), (129, 33, 65), (520, 8, 15), (520, 9, 9),
+           (600, 7, 16), (600, 7, 17), (513, 9, 33), (9, 20, 16), (9, 20, 17), (9, 20, 65), (512, 8, 8),
+           (600, 3, 9), (1500, 2, 3), (520, 1, 17), (4000, 1, 1), (2, 7000, 7)]
 
 
 def _expected(occ, cell, dtype):
