@@ -66,7 +66,7 @@ constexpr int kWaves = 4;                // tiles a block visits at once, one a 
 constexpr int kThreads = 64 * kWaves;
 constexpr int kMaxLocal = 96;            // local sweeps per visit; the tile is requeued if hit
 constexpr int kSweepChunk = 32;          // sweeps launched between host checks
-constexpr int64_t kPartMinTiles = 4096;  // grids of fewer tiles keep one queue
+constexpr int64_t kPartMinTiles = 4096;  // grids of fewer tiles keep one queue (layout_of)
 constexpr int kPartPitch = 32;           // words between the counts of 8 queues: a line each
 
 // control words after the queues (uint32); the three counts are here while
@@ -541,8 +541,12 @@ __global__ __launch_bounds__(256) void goal_yaw(FieldArgs a, const void* __restr
     out[i] = yaw;
 }
 
+constexpr int64_t kCountWords = 3 * 8 * kPartPitch;   // of eight queues
+
 struct Layout {
     int64_t d_off, open_off, mark_off, q_off, ctl_off, total;
+    int64_t part_cap;   // tiles a queue holds
+    int parts;
     uint32_t tiles;
 };
 
@@ -550,11 +554,21 @@ Layout layout_of(int nx, int ny, int nz) {
     Layout l;
     const int64_t tiles = (int64_t)((nx + kT - 1) / kT) * ((ny + kT - 1) / kT) * ((nz + kT - 1) / kT);
     l.tiles = (uint32_t)tiles;
+    // eight queues where there are tiles enough to keep them even, each with
+    // room for an eighth of the blocks that part_of deals out, whole or not. A
+    // single queue's count is one address that every visit's pushes wait for:
+    // 12 ns a visit, 3 with eight queues (4096x4096x1 voxels, a quarter solid:
+    // 162 ms a bake with one queue, 35 with eight).
+    const int64_t tx = (nx + kT - 1) / kT, ty = (ny + kT - 1) / kT, tz = (nz + kT - 1) / kT;
+    l.parts = tiles >= kPartMinTiles ? 8 : 1;
+    l.part_cap = l.parts == 8 ? ((((tx + 3) / 4) | 1) * ((ty + 1) / 2) * ((tz + 1) / 2) + 7) / 8 * 16 : tiles;
     l.d_off = 0;
     l.open_off = l.d_off + tiles * kTileVox * 4;
     l.mark_off = l.open_off + tiles * kT * 8;
     l.q_off = l.mark_off + tiles * 4;
-    l.ctl_off = l.q_off + 3 * tiles * 4;
+    // two sweeps' queues, then (eight queues) their counts right before the
+    // control words
+    l.ctl_off = l.q_off + (2 * l.parts * l.part_cap + (l.parts == 8 ? kCountWords : 0)) * 4;
     l.ctl_off = (l.ctl_off + 63) & ~(int64_t)63;
     l.total = l.ctl_off + kCtl * 4;
     return l;
@@ -623,17 +637,12 @@ SDFR_API int32_t sdfr_goal_bake(const uint8_t* occ, int32_t nx, int32_t ny, int3
     g.w1 = (float)((double)cell * sqrt(1.0));
     g.w2 = (float)((double)cell * sqrt(2.0));
     g.w3 = (float)((double)cell * sqrt(3.0));
-    // eight queues where the queue space holds them and there are tiles enough
-    // to keep them even, else one; the counts then lie right before the
-    // control words, in the queues' space
-    const int64_t part_cap = (((((int64_t)g.tx + 3) / 4) | 1) * ((g.ty + 1) / 2) * ((g.tz + 1) / 2) + 7) / 8 * 16;
-    const int64_t count_words = 3 * 8 * kPartPitch;
-    g.parts = L.tiles >= kPartMinTiles && 16 * part_cap + count_words <= 3 * (int64_t)L.tiles ? 8 : 1;
-    g.part_cap = g.parts == 8 ? (uint32_t)part_cap : L.tiles;
+    g.parts = L.parts;
+    g.part_cap = (uint32_t)L.part_cap;
     g.part_pitch = g.parts == 8 ? kPartPitch : 1;
-    g.counts = g.parts == 8 ? g.ctl - count_words : g.ctl + kCount0;
-    const int64_t shared = (g.parts == 8 ? count_words : 0) + kCtl;   // words the host reads
-    uint32_t host[3 * 8 * kPartPitch + kCtl];
+    g.counts = g.parts == 8 ? g.ctl - kCountWords : g.ctl + kCount0;
+    const int64_t shared = (g.parts == 8 ? kCountWords : 0) + kCtl;   // words the host reads
+    uint32_t host[kCountWords + kCtl];
     uint32_t* const host_ctl = host + (shared - kCtl);
     uint32_t* const host_counts = g.parts == 8 ? host : host_ctl + kCount0;
     memset(host, 0, sizeof host);

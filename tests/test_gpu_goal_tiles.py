@@ -1,7 +1,8 @@
 """The goal-field bake's tiles and queues at their edges, against the oracle's fixpoint bit for
-bit: grids of many tiles (a queue per XCD) whose sides end inside a tile, a thin one whose queue
-space holds a single queue only, one long enough for several rounds of sweeps, and the
-quantisation of voxel counts and outputs that allow no four-voxel stores."""
+bit: grids of many tiles (a queue per XCD) whose sides end inside a tile, ones a tile thick along
+each axis, either side of the tile count from which there are eight queues, one long enough for
+several rounds of sweeps, and the quantisation of voxel counts and outputs that allow no four-voxel
+stores."""
 from __future__ import annotations
 
 import ctypes
@@ -19,11 +20,16 @@ pytestmark = pytest.mark.gpu
 def _occupancy(shape, seed):
     rng = np.random.default_rng(seed)
     occ = (rng.random(shape) < 0.25).astype(np.uint8)
-    occ[shape[0] // 2, : shape[1] - 2] = 1     # a wall to go round
+    # a wall to go round
+    if shape[0] > 1:
+        occ[shape[0] // 2, : shape[1] - 2] = 1
+    else:
+        occ[:, shape[1] // 2, : shape[2] - 2] = 1
     return occ
 
 
-@pytest.mark.parametrize("shape", [(129, 131, 135), (128, 130, 136), (521, 523, 5), (3, 1030, 1029), (6, 7, 4099)],
+@pytest.mark.parametrize("shape", [(129, 131, 135), (128, 130, 136), (521, 523, 5), (3, 1030, 1029), (6, 7, 4099),
+                                   (520, 3, 515), (515, 520, 1), (1, 512, 512), (1, 512, 504)],
                          ids=str)
 def test_many_tiles_match_oracle(dev, shape):
     occ = _occupancy(shape, sum(shape))
