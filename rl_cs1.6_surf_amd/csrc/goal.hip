@@ -109,43 +109,72 @@ __device__ __forceinline__ uint32_t* queue_of(const GoalArgs& a, uint32_t k, uin
     return a.queues + ((size_t)(k & 1u) * a.parts + part) * a.part_cap;
 }
 
+// Block b runs on XCD b % 8. Kernels that walk the whole grid give each XCD a
+// contiguous eighth of their n items, as a line of the grid's rows holds several
+// tiles' voxels and is best read and written through one L2 (268 M voxels:
+// goal_init 480 -> 360 to 397 us, goal_quantise 650 -> 561). The launch is a
+// multiple of 8 blocks.
+__device__ __forceinline__ uint32_t xcd_share(uint32_t n) { return (n + 7) / 8; }
+
 // d = +inf everywhere, 0 on the free voxels of the seed box; the tiles that
 // hold a seed or touch one through their halo form the first queue. Tiles
 // without a free voxel are marked as if queued for good: no visit could lower
-// anything there. A wave a tile, a lane a column.
+// anything there. A wave a tile. A lane reads one of the tile's 64 rows, eight
+// bytes at once, whose free voxels are a byte of the tile's masks as they lie;
+// its column's seeds it takes from the rows' lanes, in the seed box's tiles
+// only. What bounds it is the bytes: 268 M voxels QQINIT us (700 with a byte a
+// lane and column, 370 a voxel a thread).
 __global__ __launch_bounds__(256) void goal_init(GoalArgs a, int lx, int ly, int lz, int hx, int hy,
                                                  int hz, int tlx, int tly, int tlz, int thx, int thy,
                                                  int thz) {
     const int lane = threadIdx.x & 63;
     uint32_t seeds = 0;
-    for (uint32_t t = blockIdx.x * 4 + (threadIdx.x >> 6); t < a.tiles; t += gridDim.x * 4) {
+    const uint32_t share = xcd_share((a.tiles + 3) / 4);
+    for (uint32_t i = blockIdx.x >> 3; i < share; i += gridDim.x >> 3) {
+        const uint32_t t = ((blockIdx.x & 7u) * share + i) * 4 + (threadIdx.x >> 6);
+        if (t >= a.tiles) break;
         const int tx = (int)(t % (uint32_t)a.tx);
         const uint32_t r = t / (uint32_t)a.tx;
         const int ty = (int)(r % (uint32_t)a.ty), tz = (int)(r / (uint32_t)a.ty);
-        const int x = tx * kT + (lane & 7), y = ty * kT + (lane >> 3), z0 = tz * kT;
-        const bool inside = x < a.nx && y < a.ny;
-        const bool box = x >= lx && x <= hx && y >= ly && y <= hy;
-        const int64_t idx = ((int64_t)z0 * a.ny + y) * a.nx + x, plane = (int64_t)a.ny * a.nx;
+        const int x0 = tx * kT, y0 = ty * kT, z0 = tz * kT;
+        uint64_t solid = ~0ull;   // bytes of row (z0 + lane / 8, y0 + lane % 8)
+        const int ry = y0 + (lane & 7), rz = z0 + (lane >> 3);
+        if (ry < a.ny && rz < a.nz) {
+            const uint8_t* o = a.occ + ((int64_t)rz * a.ny + ry) * a.nx + x0;
+            if (x0 + kT <= a.nx) {
+                __builtin_memcpy(&solid, o, 8);   // (at any alignment)
+            } else {
+                for (int b = 0; b < a.nx - x0; ++b)
+                    if (o[b] == 0) solid &= ~(0xffull << (8 * b));
+            }
+        }
+        // bit i: byte i is zero (the top bit of every non-zero byte, gathered)
+        const uint64_t low = 0x7f7f7f7f7f7f7f7full;
+        const uint64_t some = (((solid & low) + low) | solid) & ~low;
+        const uint32_t free = (uint32_t)((((some >> 7) * 0x0102040810204080ull) >> 56) ^ 0xffull);
+        ((uint8_t*)(a.open + (int64_t)t * kT))[lane] = (uint8_t)free;
+        const bool any = __any(free != 0u);
+        const bool in = tx >= tlx && tx <= thx && ty >= tly && ty <= thy && tz >= tlz && tz <= thz;
         float v[kT];
-        uint64_t mine = 0, some = 0;
 #pragma unroll
-        for (int z = 0; z < kT; ++z) {
-            const bool free = inside && z0 + z < a.nz && a.occ[idx + z * plane] == 0;
-            const bool seed = free && box && z0 + z >= lz && z0 + z <= hz;
-            const uint64_t m = __ballot(free);
-            if (lane == z) mine = m;
-            some |= m;
-            seeds += seed;
-            v[z] = seed ? 0.0f : INFINITY;
+        for (int z = 0; z < kT; ++z) v[z] = INFINITY;
+        if (in) {   // uniform
+            const int x = x0 + (lane & 7), y = y0 + (lane >> 3);
+            const bool box = x >= lx && x <= hx && y >= ly && y <= hy;
+#pragma unroll
+            for (int z = 0; z < kT; ++z) {
+                const uint32_t row = __shfl(free, z * kT + (lane >> 3));
+                const bool seed = box && z0 + z >= lz && z0 + z <= hz && ((row >> (lane & 7)) & 1u) != 0u;
+                if (seed) v[z] = 0.0f;
+                seeds += seed;
+            }
         }
         float4* col = (float4*)(a.d + (int64_t)t * kTileVox + lane * kT);
         col[0] = make_float4(v[0], v[1], v[2], v[3]);
         col[1] = make_float4(v[4], v[5], v[6], v[7]);
-        if (lane < kT) a.open[(int64_t)t * kT + lane] = mine;
         if (lane == 0) {
-            const bool in = tx >= tlx && tx <= thx && ty >= tly && ty <= thy && tz >= tlz && tz <= thz;
-            a.mark[t] = some == 0 ? ~0u : in ? 1u : 0u;
-            if (in && some) {
+            a.mark[t] = !any ? ~0u : in ? 1u : 0u;
+            if (in && any) {
                 const uint32_t part = part_of(a, tx, ty, tz);
                 queue_of(a, 1u, part)[atomicAdd(count_of(a, 1u, part), 1u)] = t;
             }
@@ -407,7 +436,8 @@ __global__ __launch_bounds__(256) void goal_reach_max(GoalArgs a) {
 // turns four tiles along x into rows of 32 voxels through LDS (rows 36 words
 // apart: the 64 columns of a wave then fall on 64 banks), so that both
 // outputs are written in whole lines, four voxels a thread (`wide`: rows and
-// outputs are aligned for it).
+// outputs are aligned for it) or one beside the next (801x803x203 voxels 256 us;
+// 272 a voxel a thread from rows of the grid). 268 M voxels 561 to 580 us by run.
 __global__ __launch_bounds__(256) void goal_quantise(GoalArgs a, double cell, float inv_quant, float quant,
                                                      uint16_t* q_out, float* g_out, int wide) {
     constexpr int kSpan = 4 * kT, kPitch = kSpan + 4;
@@ -421,7 +451,10 @@ __global__ __launch_bounds__(256) void goal_quantise(GoalArgs a, double cell, fl
     };
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const uint32_t spans = (uint32_t)(a.tx + 3) / 4u, groups = spans * (uint32_t)a.ty * (uint32_t)a.tz;
-    for (uint32_t gr = blockIdx.x; gr < groups; gr += gridDim.x) {
+    const uint32_t share = xcd_share(groups);
+    for (uint32_t i = blockIdx.x >> 3; i < share; i += gridDim.x >> 3) {
+        const uint32_t gr = (blockIdx.x & 7u) * share + i;
+        if (gr >= groups) break;   // (uniform)
         const uint32_t row = gr / spans;   // of tiles: tz * ty_count + ty
         const int tx0 = (int)(gr - row * spans) * 4;
         const int ty = (int)(row % (uint32_t)a.ty), tz = (int)(row / (uint32_t)a.ty);
@@ -433,26 +466,33 @@ __global__ __launch_bounds__(256) void goal_quantise(GoalArgs a, double cell, fl
             for (int z = 0; z < kT; ++z) s[(z * kT + (lane >> 3)) * kPitch + wave * kT + (lane & 7)] = v[z];
         }
         __syncthreads();
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            const int line = j * 32 + (int)(threadIdx.x >> 3), c = (int)(threadIdx.x & 7) * 4;
+        // line l of the LDS is the row (tz * 8 + l / 8, ty * 8 + l % 8)
+        auto place = [&](int line, int c) -> int64_t {   // of its voxel c; -1 outside the grid
             const int x = tx0 * kT + c, y = ty * kT + (line & 7), z = tz * kT + (line >> 3);
-            if (x >= a.nx || y >= a.ny || z >= a.nz) continue;
-            const int64_t i = ((int64_t)z * a.ny + y) * a.nx + x;
-            const float* v = s + line * kPitch + c;
-            if (wide) {
-                const float4 f = *(const float4*)v;
+            return x < a.nx && y < a.ny && z < a.nz ? ((int64_t)z * a.ny + y) * a.nx + x : -1;
+        };
+        if (wide) {
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                const int line = j * 32 + (int)(threadIdx.x >> 3), c = (int)(threadIdx.x & 7) * 4;
+                const int64_t at = place(line, c);
+                if (at < 0) continue;
+                const float4 f = *(const float4*)(s + line * kPitch + c);
                 const ushort4 u = make_ushort4(code(f.x), code(f.y), code(f.z), code(f.w));
-                if (q_out) *(ushort4*)(q_out + i) = u;
+                if (q_out) *(ushort4*)(q_out + at) = u;
                 if (g_out)
-                    *(float4*)(g_out + i) =
+                    *(float4*)(g_out + at) =
                         make_float4((float)u.x * quant, (float)u.y * quant, (float)u.z * quant, (float)u.w * quant);
-            } else {
-                for (int o = 0; o < 4 && x + o < a.nx; ++o) {
-                    const uint16_t u = code(v[o]);
-                    if (q_out) q_out[i + o] = u;
-                    if (g_out) g_out[i + o] = (float)u * quant;
-                }
+            }
+        } else {
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const int line = j * 8 + (int)(threadIdx.x >> 5), c = (int)(threadIdx.x & 31);
+                const int64_t at = place(line, c);
+                if (at < 0) continue;
+                const uint16_t u = code(s[line * kPitch + c]);
+                if (q_out) q_out[at] = u;
+                if (g_out) g_out[at] = (float)u * quant;
             }
         }
         __syncthreads();
@@ -650,7 +690,7 @@ SDFR_API int32_t sdfr_goal_bake(const uint8_t* occ, int32_t nx, int32_t ny, int3
     hipError_t e = hipMemcpyAsync(dev_words, host, shared * 4, hipMemcpyHostToDevice, st);
     if (e != hipSuccess) return gfail(-4, "sdfr_goal_bake: %s", hipGetErrorString(e));
     const uint32_t quads = (L.tiles + 3) / 4;   // four tiles a block
-    const int init_blocks = (int)(quads > 8192 ? 8192 : quads);
+    const int init_blocks = (int)(quads > 8192 ? 8192 : (quads + 7) / 8 * 8);
     goal_init<<<init_blocks, 256, 0, st>>>(g, lo[0], lo[1], lo[2], hi[0], hi[1], hi[2], tlo[0], tlo[1],
                                            tlo[2], thi[0], thi[1], thi[2]);
     int dev = 0, cus = 256;
@@ -680,8 +720,8 @@ SDFR_API int32_t sdfr_goal_bake(const uint8_t* occ, int32_t nx, int32_t ny, int3
     const float inv_quant = 1.0f / quant_f;
     const int wide = nx % 4 == 0 && ((uintptr_t)grid_q & 7u) == 0 && ((uintptr_t)grid & 15u) == 0;
     const int64_t groups = (int64_t)((g.tx + 3) / 4) * g.ty * g.tz;
-    goal_quantise<<<(int)(groups > 65536 ? 65536 : groups), 256, 0, st>>>(g, (double)cell, inv_quant, quant_f, grid_q,
-                                                                           grid, wide);
+    const int quantise_blocks = (int)(groups > 65536 ? 65536 : (groups + 7) / 8 * 8);
+    goal_quantise<<<quantise_blocks, 256, 0, st>>>(g, (double)cell, inv_quant, quant_f, grid_q, grid, wide);
     e = hipGetLastError();
     if (e == hipSuccess) e = hipMemcpyAsync(host_ctl, g.ctl, kCtl * 4, hipMemcpyDeviceToHost, st);
     if (e == hipSuccess) e = hipStreamSynchronize(st);

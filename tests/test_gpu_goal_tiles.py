@@ -46,6 +46,27 @@ def test_many_tiles_match_oracle(dev, shape):
         assert np.float32(field.reach_max) == ref["reach_max"]
 
 
+@pytest.mark.parametrize("nx", [1, 7, 8, 9, 15, 16, 17, 40])
+def test_occupancy_rows_at_any_alignment(dev, nx):
+    """Rows are read eight voxels at once: ends inside a tile, any address, any non-zero byte."""
+    shape = (9, 17, nx)
+    n = int(np.prod(shape))
+    rng = np.random.default_rng(nx)
+    occ = np.where(rng.random(shape) < 0.3, rng.choice([1, 2, 127, 128, 255], shape), 0).astype(np.uint8)
+    occ[0, 0, 0] = occ[8, 16, nx - 1] = 0
+    zone = {"mins": [0.5, 100.0, 50.0], "maxs": [8.0 * nx, 8.0 * 17, 8.0 * 9]}   # odd box, the last voxels in it
+    lo, hi = goalfield.seed_voxel_box(zone, np.zeros(3), 8.0, shape[::-1])
+    ref = ogoal.bake(occ, 8.0, lo, hi)
+    for offset in (0, 1, 2, 4, 7):
+        buf = torch.ones(n + 16, dtype=torch.uint8, device=dev)
+        buf[offset:offset + n] = torch.as_tensor(occ, device=dev).reshape(-1)
+        print(f"case goal rows nx={nx} offset={offset}", flush=True)
+        field = goalfield.goal_field_from_occupancy(buf[offset:offset + n].view(shape), np.zeros(3), zone, 8.0,
+                                                    device=dev)
+        assert np.array_equal(field.grid_q.cpu().numpy().view(np.uint16), ref["grid_q"])
+        assert field.bake_info["n_seed"] == ref["n_seed"]
+
+
 @pytest.mark.parametrize("shift", [0, 1])
 def test_quantised_outputs_at_any_alignment(dev, shift):
     """Through the C ABI: an odd voxel count, outputs `shift` elements into their buffers."""
