@@ -36,20 +36,34 @@ def test_empty_and_full_grids(dev):
         assert np.array_equal(got, ref.astype(np.float32)), occ.shape
 
 
-@pytest.mark.parametrize("shape", [(64, 512, 512), (256, 32, 512)])
-def test_both_pass_algorithms_match_scipy(dev, shape):
-    """Each of the y and z passes walks the parabola envelope when it has
-    many lines and searches a window per output when it has few (the switch
-    is at 512 lines per CU: 131,072 on 256 CUs). (64, 512, 512): y by window
-    (32,768 lines), z by envelope (262,144); (256, 32, 512): y by envelope
-    (131,072), z by window (16,384). Both equal scipy bit for bit."""
+@pytest.mark.parametrize("shape, density, columns", [((64, 512, 512), 0.002, True), ((256, 32, 512), 0.002, True),
+                                                     ((190, 200, 210), 2e-6, False)])
+def test_sparse_solids_match_scipy(dev, shape, density, columns):
+    """Grids of millions of voxels, few of them solid, two with a side full of solid columns: the
+    outward search of the y and z passes over few chunks and over many."""
     rng = np.random.default_rng(sum(shape))
-    occ = (rng.random(shape) < 0.002).astype(np.uint8)
-    occ[:, :, : shape[2] // 8] |= (rng.random((shape[0], shape[1], 1)) < 0.3).astype(np.uint8)
-    print(f"case edt both algorithms {shape}", flush=True)
+    occ = (rng.random(shape) < density).astype(np.uint8)
+    if columns:
+        occ[:, :, : shape[2] // 8] |= (rng.random((shape[0], shape[1], 1)) < 0.3).astype(np.uint8)
+    print(f"case edt sparse {shape}", flush=True)
     ref = edt.bake(occ, 16.0).astype(np.float32)
     got = vision.sdf_from_occupancy(occ, 16.0, device=dev, dtype=torch.float32).cpu().numpy()
     assert np.array_equal(got, ref)
+
+
+@pytest.mark.parametrize("shape", [(4100, 45, 40), (30, 8200, 30)], ids=str)
+def test_lines_past_the_lds_match_scipy(dev, shape):
+    """z lines above 4096 voxels and y lines above 8192 take the parabola envelope instead of the
+    tiles; sparse solids, so that distances reach tens of voxels and the envelope pops and walks
+    over many vertices."""
+    rng = np.random.default_rng(sum(shape))
+    for density in (1e-5, 1e-3, 0.05):
+        occ = (rng.random(shape) < density).astype(np.uint8)
+        print(f"case edt envelope {shape} density={density}", flush=True)
+        ref = edt.bake(occ, 16.0)
+        for dt, nd in ((torch.float32, np.float32), (torch.float16, np.float16)):
+            got = vision.sdf_from_occupancy(occ, 16.0, device=dev, dtype=dt).cpu().numpy()
+            assert np.array_equal(got, ref.astype(nd))
 
 
 def test_scene_occupancy_matches_scipy_and_renders(dev):
