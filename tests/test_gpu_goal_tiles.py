@@ -67,28 +67,35 @@ def test_occupancy_rows_at_any_alignment(dev, nx):
         assert field.bake_info["n_seed"] == ref["n_seed"]
 
 
-@pytest.mark.parametrize("shift", [0, 1])
-def test_quantised_outputs_at_any_alignment(dev, shift):
-    """Through the C ABI: an odd voxel count, outputs `shift` elements into their buffers."""
-    shape = (9, 11, 13)
+@pytest.mark.parametrize("nx", [12, 13, 16])
+def test_quantised_outputs_at_any_alignment(dev, nx):
+    """Through the C ABI: rows that allow four-voxel stores and rows that do not, each output some
+    elements into its buffer or not asked for, nothing written beside them."""
+    shape = (9, 11, nx)
     occ = torch.as_tensor(_occupancy(shape, 3), device=dev)
     occ[0, 0, 0] = 0
     n = occ.numel()
     lib = _sdfr.load()
     lo = (ctypes.c_int32 * 3)(0, 0, 0)
     ref = ogoal.bake(occ.cpu().numpy(), 16.0, np.zeros(3, np.int32), np.zeros(3, np.int32))
-    ws = torch.empty(int(lib.sdfr_goal_workspace_bytes(13, 11, 9)), dtype=torch.uint8, device=dev)
-    q = torch.zeros(n + 8, dtype=torch.int16, device=dev)
-    g = torch.zeros(n + 8, dtype=torch.float32, device=dev)
+    ws = torch.empty(int(lib.sdfr_goal_workspace_bytes(nx, 11, 9)), dtype=torch.uint8, device=dev)
     info = _sdfr.GoalInfo()
-    print(f"case goal alignment {shift}", flush=True)
-    rc = lib.sdfr_goal_bake(occ.data_ptr(), 13, 11, 9, 16.0, lo, lo, 1 << 20, q[shift:].data_ptr(),
-                            g[shift:].data_ptr(), ctypes.byref(info), ws.data_ptr(), ws.numel(),
-                            torch.cuda.current_stream().cuda_stream)
-    assert rc == 0
-    assert np.array_equal(q[shift:shift + n].cpu().numpy().view(np.uint16).reshape(shape), ref["grid_q"])
-    assert np.array_equal(g[shift:shift + n].cpu().numpy().reshape(shape), ref["grid"])
-    assert not q[shift + n:].any() and not g[shift + n:].any() and not q[:shift].any()
+    for qs, gs in [(a, b) for a in (0, 1, 2, 3, None) for b in (0, 1, 2, 3, None) if (a, b) != (None, None)]:
+        q = torch.full((n + 8,), 77, dtype=torch.int16, device=dev)
+        g = torch.full((n + 8,), -1.0, dtype=torch.float32, device=dev)
+        print(f"case goal alignment nx={nx} q={qs} grid={gs}", flush=True)
+        rc = lib.sdfr_goal_bake(occ.data_ptr(), nx, 11, 9, 16.0, lo, lo, 1 << 20,
+                                None if qs is None else q[qs:].data_ptr(), None if gs is None else g[gs:].data_ptr(),
+                                ctypes.byref(info), ws.data_ptr(), ws.numel(),
+                                torch.cuda.current_stream().cuda_stream)
+        assert rc == 0
+        for out, s, want, guard in ((q.cpu().numpy(), qs, ref["grid_q"].view(np.int16), 77),
+                                    (g.cpu().numpy(), gs, ref["grid"], -1.0)):
+            if s is None:
+                assert (out == guard).all()
+                continue
+            assert np.array_equal(out[s:s + n].reshape(shape), want)
+            assert (out[:s] == guard).all() and (out[s + n:] == guard).all()
 
 
 @pytest.mark.parametrize("shape", [(24, 24, 40), (17, 23, 33), (8, 8, 4), (1, 1, 36)], ids=str)

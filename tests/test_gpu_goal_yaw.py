@@ -49,6 +49,39 @@ def test_matches_the_samples_formula(dev, n, quant):
         assert np.minimum(diff, 360.0 - diff).max() < 1e-4
 
 
+def test_samples_and_yaws_run_on_the_current_stream(dev):
+    """On a side stream behind the work that makes their positions, and captured into a graph,
+    which a launch on any other stream would not enter: replayed on new positions, with eager calls
+    between the replays."""
+    field, mins = _field(dev, False)
+    rng = np.random.default_rng(1)
+    p = [torch.as_tensor(mins + rng.uniform(0.0, 1.0, (300, 3)) * np.array(field.dims) * field.cell, device=dev)
+         for _ in range(4)]
+    want = [(field.sample(x), field.descent_yaw(x)) for x in p]
+    torch.cuda.synchronize()
+    side = torch.cuda.Stream(dev)
+    print("case goal field on a side stream", flush=True)
+    with torch.cuda.stream(side):
+        big = torch.randn(4096, 4096, device=dev)
+        for _ in range(10):
+            big = big @ big * 1e-3
+        pos = p[0] + (big[0, 0] * 0.0).double().nan_to_num()
+        got = field.sample(pos), field.descent_yaw(pos)
+    side.synchronize()
+    assert all(torch.equal(a, b) for a, b in zip(got, want[0]))
+    pos = p[0].clone()
+    graph = torch.cuda.CUDAGraph()
+    print("case goal field captured", flush=True)
+    with torch.cuda.graph(graph):
+        out = field.sample(pos), field.descent_yaw(pos)
+    for x, w in zip(p[1:], want[1:]):
+        pos.copy_(x)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(out, w))
+        assert torch.equal(field.sample(x), w[0])
+
+
 def test_no_positions_are_refused(dev):
     field, _ = _field(dev, False)
     with pytest.raises(RuntimeError):
