@@ -314,7 +314,9 @@ SDFR_API const char* sdfr_edt_last_error(void);
  * Outputs (either may be NULL, not both): grid_q, the uint16 grid of the
  * reference's cache file; grid, its f32 dequantisation u16 * quant (what
  * GoalField holds). `workspace`: sdfr_goal_workspace_bytes() bytes of device
- * memory, 64-byte aligned. Synchronises `stream` (the host reads the
+ * memory, 64-byte aligned: ~4.2 per voxel of the grid rounded up to whole tiles
+ * of 8x8x8 voxels (so 8 times that of its own voxels for a grid one voxel
+ * thick). Synchronises `stream` (the host reads the
  * wavefront's queue length every few sweeps). Returns 0; -5 no free seed
  * voxel, -6 sentinel beyond the uint16 range, -7 not converged within
  * max_sweeps (sdfr_goal_last_error()). */

@@ -26,8 +26,9 @@
 // edt_slabs; one thread per y or z line).
 //
 // Scratch: two int32 planes of the grid and one uint64 envelope stack per
-// line (~16 bytes per voxel, sdfr_edt_workspace_bytes); the tiles use at most
-// 13 bytes per voxel of it.
+// line (~16 bytes per voxel, sdfr_edt_workspace_bytes); the tiles use 2.25 bytes
+// per voxel of it in long rows of up to 509 planes, 12 at most (rows of one
+// voxel).
 
 #include <hip/hip_runtime.h>
 #include <hip/hip_fp16.h>
@@ -232,7 +233,7 @@ __global__ __launch_bounds__(256) void edt_slabs(const int32_t* __restrict__ f, 
 }
 
 // ------------------------------------------------------------- tiled passes --
-// The transform in three kernels that move 7.5 bytes a voxel and the output
+// The transform in three kernels that move 5.5 bytes a voxel and the output
 // between them (a byte of occupancy, a quarter byte of packed bits each way,
 // 16-bit squares each way). A pass searches, for every output q of a line,
 // D(q) = min over p of f(p) + (q - p)^2 over whole lines staged in LDS.
@@ -256,15 +257,27 @@ __global__ __launch_bounds__(256) void edt_slabs(const int32_t* __restrict__ f, 
 //     agree about both, so on the scenes measured a wave searches ~4 of a
 //     line's 128 chunks.
 //
-// What bounds it is vector issue (the searches) and, at their start, the wait
-// for the tile: at 256x256x128 voxels 5.5 + 32 + 26 us (36 + 98 + 62 us for a
-// wave per row and a search per output), at 1024x1024x256 125 + 750 + 622 us
-// (3049 + 4881 + 3207 us for the wave per row and the walk per line); the
-// bytes alone take 14 and 430 us at a copy's 4.7 TB/s. 8 outputs a thread
-// beat 16 (40 + 32, 887 + 831 us) as they leave twice the waves in flight;
-// tiles 32 words wide beat 64, of which fewer fit a CU (33 + 27, 1077 +
-// 785 us); 1024 threads beat 512 in the y pass, whose tiles fill the LDS
-// (749 against 930 us), and lose in the z pass (741 against 622).
+// What bounds it: at 1024x1024x256 voxels (125 + 755 + 622 us; 3049 + 4881 +
+// 3207 for a wave per row and a walk per line) vector issue, 60, 69 and 85% of
+// the cycles in the packing, y and z passes, and in the y pass the waits for its
+// tiles besides. At 256x256x128 (6 + 31 + 26 us; 36 + 98 + 62 for a wave per row
+// and a search per output) all tiles are in flight at once, vector issue is 14,
+// 38 and 41%, and a wave spends 40% of its time waiting for its tile and its
+// group and 36% for its turn at the SIMD; LDS is busy 4% of the time, without a
+// bank conflict. The bytes alone take 410 and 16 us at a copy's 4.9 TB/s. 8
+// outputs a thread beat 16 (40 + 32, 887 + 831 us) as they leave twice the waves
+// in flight (2 in small grids: small_grid); tiles 32 words wide beat 64, of which
+// fewer fit a CU (33 + 27, 1077 + 785 us); 1024 threads beat 512 in the y pass,
+// whose tiles fill the LDS (749 against 930 us), and lose in the z pass (741
+// against 622).
+//
+// The walk per line that the tiles replaced (a search per output for few lines)
+// was timed against them on grids of 64x64x300 to 1024^3 voxels, empty, with a
+// floor and boxes, and with one voxel in 10^5 and in 100 solid: the tiles win on
+// all, by least on empty cubes in 32 bits (640^3 9.1 -> 4.5 ms, 1024^3 47.7 ->
+// 23.9), and also with one narrow tile a CU (z lines of 4000 voxels: 300x300x4000
+// 13.7 -> 4.8 ms; y lines of 8000: 200x8000x300 21 -> 3.4 ms), so only the lines
+// that do not fit walk.
 typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
 
 constexpr int kBlk = 8;       // outputs a thread takes and rows a chunk holds, ...
@@ -419,7 +432,7 @@ struct PassArgs {
     int pitch;
     void* out;             // y pass: the plane; z pass: the distances
     int nx, ny, nz, words;
-    int n, blks;           // line length and its 16-output blocks
+    int n, blks;           // line length and its blocks of BLK rows
     int tiles;             // tiles along x
     int64_t blocks;
     double cell2;

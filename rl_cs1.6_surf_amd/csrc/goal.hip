@@ -224,17 +224,21 @@ __device__ __forceinline__ void wave_sync() {
 // lines; rows of the grid took 28 loads and 240 lines), and the free voxels
 // are lane masks in scalar registers.
 //
-// What bounds it: in the ~20 long sweeps of a bake (up to 5000 visits, one a
-// wave) vector issue and LDS reads of the ~10 relaxations of a visit, in the
-// ~30 short ones the chain of round trips to memory of one visit (queue, tile,
-// mark, slot: ~6 us). 256x256x128 voxels, 50 sweeps: 29 us a sweep with a block
-// of 512 threads and 26 LDS reads a voxel, 18 with a wave a tile, 16 with the
-// columns loaded straight to their lanes; a whole bake 1086 us with a queue
-// per XCD, 887 with the distances by tile, 840 with the halo's loads under a
-// branch and the pass down z as selects. Also measured: flags per tile instead
-// of queues (no claims, but a static deal of tiles to waves: 28 us a sweep),
-// reading a mark before its atomic (+2 us), no order along z (+2 us), queueing
-// only tiles whose halo copy would fall (20% fewer visits, each 3 us longer).
+// What bounds it: the time of the slowest visits. In a bake of a closed scene of
+// 256x256x128 voxels (50 sweeps, up to 23 us each) no unit is near its limit in
+// any sweep: vector issue is busy 28% of the cycles at most and LDS 14% (a sixth
+// of it conflicts). In the ~20 long sweeps (up to 5000 visits, one a wave) a wave
+// spends 42% of its time waiting for memory and LDS and 31% for its turn at the
+// SIMD, over the ~10 relaxations of a visit; in the ~30 short ones it is the
+// chain of round trips to memory of one visit (queue, tile, mark, slot: ~6 us).
+// 29 us a sweep with a block of 512 threads and 26 LDS reads a voxel, 18 with a
+// wave a tile, 16 with the columns loaded straight to their lanes; a whole bake
+// of that scene 1086 us with a queue per XCD, 887 with the distances by tile, 840
+// to 917 by run with the halo's loads under a branch and the pass down z as
+// selects. Also measured: flags per tile instead of queues (no claims, but a
+// static deal of tiles to waves: 28 us a sweep), reading a mark before its atomic
+// (+2 us), no order along z (+2 us), queueing only tiles whose halo copy would
+// fall (20% fewer visits, each 3 us longer).
 __global__ __launch_bounds__(kThreads) void goal_sweep(GoalArgs a, const uint64_t* __restrict__ open_planes,
                                                        uint32_t k) {
     __shared__ __align__(16) float s_all[kWaves][kTileLds];
